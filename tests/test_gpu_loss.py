@@ -201,3 +201,16 @@ def test_forward_fused_l1_rejects_other_passes():
     with pytest.raises(ValueError):
         va.render(cam, w.img_size, t, s, o, pass_=va.RasterPass.BACKWARD, l1_target=gtp,
                   render_mode=va.SplatRenderMode.SURFEL)
+
+
+@pytest.mark.parametrize("h,w,cn,opts", [
+    (1, 1, 4, dict(mask=True, alpha_weight=0.2)), (5, 64, 3, dict()), (16, 65, 4, dict(alpha_weight=0.3)),
+    (17, 63, 3, dict(mask=True)), (33, 59, 4, dict(composite_bg=(0.1, 0.9, 0.4), alpha_weight=0.1)),
+    (15, 133, 4, dict(mask=True)), (1040, 2753, 4, dict(mask=True, alpha_weight=0.1)), (2161, 3845, 3, dict()),
+])
+def test_loss_strips(h, w, cn, opts):
+    """The 64-column strips' edges (a column or a row alone, one lane past a
+    strip, halo columns cut on either side), with strips of 16 rows (the small
+    images) and of several tile rows (the two large ones)."""
+    pred, gt = _case(h, w, cn, h + w)
+    _check(pred, gt, opts, "partials" if h < 100 else "scalar")
