@@ -259,7 +259,14 @@ vs_status vs_ctx_set_validation(vs_ctx* ctx, int enable);
  * shortened list, and the geometry render's median-id channel is an index
  * into that list (the same position within its tile's list).
  * num_intersections still reports every intersection; the state view gives
- * the listed ones. */
+ * the listed ones.
+ * With VS_CUTOFF_OFF everything a caller sees is the full lists', but a render
+ * whose tiles list 2048 intersections or more on average does not build them:
+ * it rasterises from lists the cutoff shortened, counts the full lists'
+ * offsets for tile_offsets without emitting them, and vs_fwd_state_view builds
+ * the full lists when it is first called on the state.  A lagged render of
+ * that kind whose capacity overflows drops only what its short lists cannot
+ * hold (usually nothing); its counts and offsets are the full lists'. */
 typedef enum vs_cutoff_mode { VS_CUTOFF_AUTO = 0, VS_CUTOFF_OFF = 1, VS_CUTOFF_ON = 2 } vs_cutoff_mode;
 vs_status vs_ctx_set_depth_cutoff(vs_ctx* ctx, vs_cutoff_mode mode);
 

@@ -222,3 +222,60 @@ def test_cutoff_auto_turns_on_for_long_lists(ctx):
             assert v.listed_intersections == v.num_intersections
         out.state.free()
         del t, s, o
+
+
+@pytest.mark.parametrize("n,size,focal,pass_name,mode_name,lagged", [
+    (320_000, (250, 170), 195.0, "BACKWARD", "DEFAULT", False), (320_000, (1111, 35), 868.0, "BACKWARD", "MIP", True),
+    (900_000, (161, 150), 30.0, "BACKWARD_SMOOTH_CUTOFF", "DEFAULT", False),
+    (320_000, (250, 170), 195.0, "FORWARD", "DEFAULT", False),
+])
+def test_long_lists_with_the_cutoff_off(ctx, n, size, focal, pass_name, mode_name, lagged):
+    """With the cutoff off, renders whose tiles list 2048 pairs or more on
+    average build short lists internally: the caller's tile offsets, the state
+    view's lists and ranges (built when asked for), counts, image, visibility
+    and gradients are the oracle's full lists', with one and with several
+    64-column spans of tiles and with empty tiles at the image's edge."""
+    pass_, mode = va.RasterPass[pass_name], va.SplatRenderMode[mode_name]
+    sc = scenes.scene_c4(n)
+    cam = va.Camera.from_focal(focal, focal, size).uniforms(size)
+    t, s, o = to_gpu(sc)
+    print(f"[case] cutoff off, long lists n={n} {size} f={focal} {pass_name} {mode_name} lagged={lagged}", flush=True)
+    flags = (po.FLAG_BWD_INFO if pass_.bwd_info() else 0) | (po.FLAG_MIP if mode == va.SplatRenderMode.MIP else 0)
+    flags |= po.FLAG_SMOOTH_CUTOFF if pass_ == va.RasterPass.BACKWARD_SMOOTH_CUTOFF else 0
+    ref = po.render_forward(cam, size, sc.transforms, sc.sh_coeffs, sc.raw_opacities, flags=flags)
+    t_count = ((size[0] + 15) // 16) * ((size[1] + 15) // 16)
+    assert ref.info.num_intersections >= 2048 * t_count, ref.info.num_intersections / t_count
+    if lagged:
+        va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode).state.free()
+        ctx.set_lagged_counts(True)
+    out = va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode)
+    torch.cuda.synchronize()
+    offsets = out.aux.tile_offsets.cpu().numpy().reshape(-1, 2).view(np.uint32)
+    if not pass_.bwd_info():
+        np.testing.assert_array_equal(offsets, ref.get(po.F_TILE_OFFSETS).reshape(-1, 2))
+        ctx.set_depth_cutoff(ctx.CUTOFF_ON)
+        cut = va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode)
+        assert torch.equal(out.out_img, cut.out_img)
+        return
+    np.testing.assert_array_equal(offsets, ref.get(po.F_TILE_OFFSETS_SHRUNK).reshape(-1, 2))
+    img = out.out_img.cpu().numpy()
+    assert np.array_equal(img.view(np.uint32), ref.get(po.F_OUT_IMG).view(np.uint32))
+    np.testing.assert_array_equal(out.aux.visible.cpu().numpy(), ref.get(po.F_VISIBLE))
+    for after_view in (False, True):        # the view leaves the state as the backward needs it
+        if after_view:
+            gpu = gpu_state_arrays(out)
+            total = ref.info.num_intersections
+            assert gpu["view"].depth_cutoff == 0 and gpu["view"].listed_intersections >= total
+            np.testing.assert_array_equal(gpu["counts"], ref.get(po.F_INTERSECT_COUNTS))
+            np.testing.assert_array_equal(gpu["listed_counts"], gpu["counts"])
+            np.testing.assert_array_equal(gpu["tile"][:total], ref.get(po.F_ISECT_TILE))
+            np.testing.assert_array_equal(gpu["gid"][:total], ref.get(po.F_ISECT_GID))
+            np.testing.assert_array_equal(gpu["ranges"].reshape(-1, 2), ref.get(po.F_TILE_OFFSETS).reshape(-1, 2))
+        rng = np.random.default_rng(5)
+        v_out = (rng.standard_normal(img.shape) / img.size).astype(np.float32)
+        g = va.render_backward(out, t, s, o, torch.from_numpy(v_out).cuda())
+        rg = ref.backward(v_out)
+        vc = g.v_combined.cpu().numpy()
+        for k0, k1, name in ((0, 2, "v_xy"), (2, 5, "v_conic"), (5, 8, "v_rgb"), (8, 9, "v_opacity"), (9, 10, "v_refine")):
+            _check_grads(vc[:, k0:k1], rg["v_combined"][:, k0:k1], name)
+    out.state.free()

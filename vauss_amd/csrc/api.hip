@@ -140,6 +140,14 @@ struct vs_fwd_state {
     bool cutoff = false;
     uint32_t* listed = nullptr;
     uint32_t* kept_counts = nullptr;
+    // the cutoff stands in for the full lists (VS_CUTOFF_OFF, long lists):
+    // everything the caller sees is the full lists'; the state view builds
+    // them when it is first asked
+    bool hidden = false;
+    mutable void* view_arena = nullptr;
+    mutable uint32_t* view_tiles = nullptr;
+    mutable uint32_t* view_gids = nullptr;
+    mutable uint32_t* view_ranges = nullptr;
 };
 
 namespace {
@@ -547,6 +555,7 @@ extern "C" vs_status vs_ctx_stage_times(vs_ctx* c, vs_stage_times* out) {
 extern "C" void vs_fwd_state_free(vs_fwd_state* st) {
     if (!st) return;
     hipSetDevice(st->ctx->device);
+    lib_free(st->ctx, st->view_arena);
     lib_free(st->ctx, st->isect_arena);
     lib_free(st->ctx, st->arena);
     delete st;
@@ -812,10 +821,20 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
     // Depth cutoff (gaussian modes): per-tile tables of (bh x CUT_BINS x (bw + 1))
     // u32 masses (then their sums over rows) and u16 prefix counts, at most 256 MiB.
     const uint64_t cut_words = (uint64_t)st->tbh * CUT_BINS * ((uint64_t)st->tbw + 1u);
-    bool cutoff = false;
-    if (!surfel && N > 0 && I > 0 && st->tbw <= CUT_MAX_BW && cut_words * 6u <= (256ull << 20) &&
-        ctx->depth_cutoff != VS_CUTOFF_OFF)
-        cutoff = ctx->depth_cutoff == VS_CUTOFF_ON || (uint64_t)I >= (uint64_t)CUT_AUTO_PER_TILE * T;
+    // With the cutoff off, a render whose tiles list CUT_AUTO_PER_TILE pairs or
+    // more on average takes it all the same, hidden: the caller's outputs are
+    // the full lists' (their offsets counted without building them), and the
+    // state view builds the lists if it is asked for.  Geometry passes, whose
+    // median channel indexes the lists, keep them.
+    const bool tables = !surfel && N > 0 && I > 0 && st->tbw <= CUT_MAX_BW && cut_words * 6u <= (256ull << 20);
+    const bool heavy = (uint64_t)I >= (uint64_t)CUT_AUTO_PER_TILE * T;
+    const uint32_t count_words = tables ? tile_count_words(st->tbw, st->tbh) : 0u;
+    const bool hidden = tables && heavy && ctx->depth_cutoff == VS_CUTOFF_OFF && !geometry &&
+                        count_words * 4u <= TILE_COUNT_MAX_LDS;
+    const bool cutoff = hidden || (tables && (ctx->depth_cutoff == VS_CUTOFF_ON ||
+                                              (ctx->depth_cutoff == VS_CUTOFF_AUTO && heavy)));
+    st->hidden = hidden;
+    uint32_t* full_start = nullptr;      // hidden: [T + 1] the full lists' starts
     st->cutoff = cutoff;
     hipEvent_t sort_done = nullptr;   // exact renders: the sorts' flag readback
     struct EventBack { vs_ctx* c; hipEvent_t& e; ~EventBack() { if (e) c->pool.push_back(e); } } sort_done_back{ctx, sort_done};
@@ -836,6 +855,9 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
         const size_t o_pend = cutoff ? itake((size_t)st->tbh * ((size_t)st->tbw + 1u) * 4) : 0;
         const size_t o_kblk = cutoff ? itake((size_t)nblocks * 4) : 0;
         const size_t o_ptot = cutoff ? itake(4) : 0;
+        const size_t o_diff = hidden ? itake(((size_t)st->tbw + 1u) * st->tbh * 4) : 0;
+        const size_t o_fstart = hidden ? itake(((size_t)T + 1u) * 4) : 0;
+        const size_t o_fpart = hidden ? itake((size_t)tile_count_groups(N) * count_words * 4) : 0;
         // serves both sorts (the depth sort on 9-bit digits, the tile sort on tile_rb-bit ones)
         const uint32_t tile_rb = tile_radix_bits(tile_bits);
         const size_t o_tmp = itake(std::max(sort_tmp_bytes(I, false, tile_rb), sort_tmp_bytes(M, false, DEPTH_RADIX_BITS)));
@@ -890,6 +912,17 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
             // the emitters are the splats that keep a pair: their count stays on the device
             VS_HIP(launch_scan_blocks(ca.kept_blocks, nblocks, st->counters + CNT_KEPT, s), "cutoff emitter offsets");
             m_dev = st->counters + CNT_KEPT;
+        }
+        if (hidden && out->tile_offsets) {
+            StageTimer tm(ctx, ST_EMIT);
+            TileCountArgs ta{};
+            ta.num_splats = N; ta.tile_bw = st->tbw; ta.tile_bh = st->tbh; ta.counts = st->counts; ta.proj = st->proj;
+            ta.partial = reinterpret_cast<uint32_t*>(ib + o_fpart);
+            ta.diff = reinterpret_cast<int32_t*>(ib + o_diff);
+            ta.start = full_start = reinterpret_cast<uint32_t*>(ib + o_fstart);
+            VS_HIP(launch_fill_u32(reinterpret_cast<uint32_t*>(ta.diff), 0u, ((uint64_t)st->tbw + 1u) * st->tbh, s),
+                   "zero tile counts");
+            VS_HIP(launch_tile_counts(ta, s), "tile counts");
         }
         const uint32_t* slot_counts = cutoff ? st->kept_counts : st->counts;
         {
@@ -965,7 +998,7 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
         // (no copy behind the forward)
         VS_HIP(launch_tile_order(st->ranges, T, st->tile_order, s, bwd_info ? st->ranges_shrunk : nullptr, true,
                                  ctx->dev_flags, lag_slot ? lag_slot->host + CNT_COUNT : nullptr, CTX_FLAGS,
-                                 out->tile_offsets),
+                                 out->tile_offsets, nullptr, 0, full_start),
                "tile order");
         ra.order = st->tile_order;
         ra.bg_r = background[0]; ra.bg_g = background[1]; ra.bg_b = background[2];
@@ -1280,9 +1313,85 @@ extern "C" vs_status vs_geo_zero_rows(vs_ctx* ctx, uint32_t* words, uint64_t num
     return VS_OK;
 }
 
+// The full lists of a render that took the cutoff hidden, into buffers of the
+// state's own (its short lists stay as the backward reads them): the stages a
+// render with short lists runs, on the counts and rows the state keeps.  Waits
+// for the stream.
+static vs_status build_full_lists(const vs_fwd_state* st) {
+    vs_ctx* ctx = st->ctx;
+    VS_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    hipStream_t s = ctx->stream;
+    uint32_t hc[CNT_COUNT];
+    VS_HIP(hipMemcpyAsync(hc, st->counters, sizeof(hc), hipMemcpyDeviceToHost, s), "counter readback");
+    VS_HIP(hipStreamSynchronize(s), "hipStreamSynchronize");
+    const uint32_t N = st->N, T = st->T, I = st->I, M = hc[CNT_EMITTERS];
+    uint64_t I64 = 0;
+    std::memcpy(&I64, hc + CNT_ISECT64, 8);
+    const uint32_t n = (uint32_t)std::min<uint64_t>(I64, I);        // a lagged render's arena may hold fewer
+    const uint32_t depth_bits = hc[CNT_VISIBLE] ? bit_length((uint64_t)(hc[CNT_DEPTH_MAX] - hc[CNT_DEPTH_MIN])) : 0u;
+    const uint32_t tile_bits = bit_length(T), tile_rb = tile_radix_bits(tile_bits), nblocks = (N + 255) / 256;
+    size_t off = 0;
+    auto take = [&](size_t bytes) { const size_t o = off; off += align256(bytes); return o; };
+    const size_t o_tiles = take((size_t)I * 4), o_gids = take((size_t)I * 4), o_rng = take((size_t)T * 8);
+    const size_t o_tu = take((size_t)I * 4), o_vu = take((size_t)I * 4);
+    const size_t o_dk = take((size_t)M * 4), o_dv = take((size_t)M * 4), o_dks = take((size_t)M * 4);
+    const size_t o_ord = take((size_t)M * 4), o_base = take((size_t)(M + 1) * 4), o_base_g = take((size_t)N * 4);
+    const size_t o_scan = take(scan_lookback_status_words(M) * 4), o_tord = take((size_t)8 * ((T + 7) / 8) * 4);
+    const size_t o_tmp = take(std::max(sort_tmp_bytes(I, false, tile_rb), sort_tmp_bytes(M, false, DEPTH_RADIX_BITS)));
+    void* arena = nullptr;
+    VS_HIP(lib_alloc(ctx, &arena, off, s), "hipMallocAsync(full lists)");
+    struct Back { vs_ctx* c; void*& p; ~Back() { if (p) lib_free(c, p); } } back{ctx, arena};
+    char* b = static_cast<char*>(arena);
+    auto u32 = [&](size_t o) { return reinterpret_cast<uint32_t*>(b + o); };
+    uint32_t* err = ctx->dev_flags + FLAG_SORT_STALL;
+    const SortZeroSpan depth_zero = sort_zero_span(M, 0, depth_bits, b + o_tmp, DEPTH_RADIX_BITS);
+    const SortZeroSpan tile_zero = sort_zero_span(n, 0, tile_bits, b + o_tmp, tile_rb);
+    VS_HIP(launch_ranges_init(u32(o_rng), T, s), "range init");
+    if (M > 0 && n > 0) {
+        CompactArgs ca{};
+        ca.num_splats = N; ca.counts = st->counts; ca.depth_bits = st->depth_bits;
+        ca.block_offsets = st->block_stats + (size_t)BS_EMIT * nblocks;
+        ca.counters = st->counters;
+        ca.keys = u32(o_dk); ca.vals = u32(o_dv);
+        ca.zero = depth_zero.ptr; ca.zero_words = depth_zero.words;
+        ca.zero2 = u32(o_scan); ca.zero2_words = scan_lookback_status_words(M);
+        VS_HIP(launch_compact(ca, s), "compaction");
+        VS_HIP(radix_sort_pairs(u32(o_dk), u32(o_dv), u32(o_dks), u32(o_ord), M, nullptr, false, 0, depth_bits, b + o_tmp, err, s,
+                                ctx->spin_limit, nullptr, depth_zero.ptr != nullptr, DEPTH_RADIX_BITS, nullptr),
+               "depth sort");
+        VS_HIP(scan_u32_lookback(st->counts, u32(o_base), M, u32(o_scan), err, s, ctx->spin_limit, u32(o_ord), nullptr, N,
+                                 u32(o_base_g), true, EMIT_SMALL_LIST), "slot scan");
+        EmitArgs ea{};
+        ea.num_splats = N; ea.tile_bw = st->tbw; ea.tile_bh = st->tbh;
+        ea.num_emitters = M; ea.order = u32(o_ord);
+        ea.counts = st->counts; ea.slot_base = u32(o_base); ea.slot_base_g = u32(o_base_g);
+        ea.zero = tile_zero.ptr; ea.zero_words = tile_zero.words;
+        ea.proj = st->proj; ea.tiles = u32(o_tu); ea.vals = u32(o_vu); ea.capacity = n;
+        VS_HIP(launch_emit(ea, s), "emit kernel");
+        TileRangesOut tro{u32(o_rng), T, false};
+        VS_HIP(radix_sort_pairs(u32(o_tu), u32(o_vu), u32(o_tiles), u32(o_gids), n, nullptr, false, 0, tile_bits, b + o_tmp, err, s,
+                                ctx->spin_limit, &tro, tile_zero.ptr != nullptr, tile_rb), "tile sort");
+        if (!tro.done) VS_HIP(launch_tile_ranges(u32(o_tiles), n, T, u32(o_rng), s, nullptr), "tile ranges");
+        VS_HIP(launch_tile_order(u32(o_rng), T, u32(o_tord), s, nullptr, true), "empty tiles");
+    } else {
+        VS_HIP(launch_tile_order(u32(o_rng), T, u32(o_tord), s, nullptr, true), "empty tiles");
+    }
+    VS_HIP(launch_tiles_from_ranges(u32(o_rng), T, I, u32(o_tiles), s), "tile ids from ranges");
+    vs_status fe = sync_sort_flag(ctx);
+    if (fe != VS_OK) return fe;
+    st->view_tiles = u32(o_tiles); st->view_gids = u32(o_gids); st->view_ranges = u32(o_rng);
+    st->view_arena = arena;
+    arena = nullptr;      // the state's now
+    return VS_OK;
+}
+
 extern "C" vs_status vs_fwd_state_view(const vs_fwd_state* st, vs_state_view* o) {
     if (!st || !o) return fail(VS_ERR_INVALID, "null argument");
-    if (st->tiles_pending && st->I > 0) {
+    if (st->hidden && !st->view_arena) {
+        vs_status ve = build_full_lists(st);
+        if (ve != VS_OK) return ve;
+    }
+    if (!st->hidden && st->tiles_pending && st->I > 0) {
         vs_ctx* ctx = st->ctx;
         VS_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         VS_HIP(launch_tiles_from_ranges(st->ranges, st->T, st->I, st->tiles, ctx->stream), "tile ids from ranges");
@@ -1301,10 +1410,12 @@ extern "C" vs_status vs_fwd_state_view(const vs_fwd_state* st, vs_state_view* o)
     o->proj_aux = reinterpret_cast<const float*>(st->proj_aux);
     o->proj_surf = reinterpret_cast<const float*>(st->proj_surf);
     o->tile_ranges = st->ranges;
+    if (st->hidden) { o->isect_tiles = st->view_tiles; o->isect_gids = st->view_gids; o->tile_ranges = st->view_ranges; }
+    const bool cut = st->cutoff && !st->hidden;
     o->listed_intersections = st->I;
-    o->depth_cutoff = st->cutoff ? 1u : 0u;
-    o->listed_counts = st->cutoff ? st->kept_counts : st->counts;
-    if (st->cutoff && st->listed) {
+    o->depth_cutoff = cut ? 1u : 0u;
+    o->listed_counts = cut ? st->kept_counts : st->counts;
+    if (cut && st->listed) {
         vs_ctx* ctx = st->ctx;
         VS_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         uint32_t listed = 0;

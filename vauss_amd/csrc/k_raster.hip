@@ -110,7 +110,8 @@ __global__ void __launch_bounds__(ORDER_BLOCK) tile_order_kernel(uint32_t* range
                                                                  const uint32_t* __restrict__ flags_from,
                                                                  uint32_t* flags_to, uint32_t nflags,
                                                                  uint32_t* __restrict__ aux_out,
-                                                                 float* __restrict__ zero, uint64_t zero_floats) {
+                                                                 float* __restrict__ zero, uint64_t zero_floats,
+                                                                 const uint32_t* __restrict__ full_start) {
     // Blocks past the eight bands clear `zero` (8-byte aligned; the backward's
     // gradient rows), which would otherwise take a launch of its own.
     if (blockIdx.x >= 8u) {
@@ -143,8 +144,14 @@ __global__ void __launch_bounds__(ORDER_BLOCK) tile_order_kernel(uint32_t* range
             shrunk_init[2 * t + 1] = lo;
         }
         if (aux_out) {
-            aux_out[2 * t] = lo;
-            aux_out[2 * t + 1] = shrunk_init ? lo : hi;
+            uint32_t alo = lo, ahi = hi;
+            if (full_start) {
+                alo = full_start[t];
+                ahi = full_start[t + 1];
+                if (ahi <= alo) alo = ahi = 0u;
+            }
+            aux_out[2 * t] = alo;
+            aux_out[2 * t + 1] = shrunk_init ? alo : ahi;
         }
     }
     __syncthreads();
@@ -622,7 +629,9 @@ __global__ void __launch_bounds__(FWD_BATCH) raster_fwd_kernel(RasterArgs a) {
     if constexpr (BWD) {
         if (l == 0 && last > lo) {
             atomicMax(&a.ranges_shrunk[tile * 2 + 1], last);
-            if (a.aux_ranges) atomicMax(&a.aux_ranges[tile * 2 + 1], last);
+            // the caller's range ends as far past its own start, which indexes
+            // the full list where `ranges` holds its front alone
+            if (a.aux_ranges) atomicMax(&a.aux_ranges[tile * 2 + 1], a.aux_ranges[tile * 2] + (last - lo));
         }
     }
 }
@@ -1233,7 +1242,8 @@ hipError_t launch_tile_ranges(const uint32_t* tiles, uint32_t n, uint32_t num_ti
 
 hipError_t launch_tile_order(uint32_t* ranges, uint32_t num_tiles, uint32_t* order, hipStream_t s,
                              uint32_t* shrunk_init, bool fix_empty, const uint32_t* flags_from, uint32_t* flags_to,
-                             uint32_t nflags, uint32_t* aux_out, float* zero, uint64_t zero_floats) {
+                             uint32_t nflags, uint32_t* aux_out, float* zero, uint64_t zero_floats,
+                             const uint32_t* full_start) {
     if (num_tiles == 0) return hipSuccess;
     if (!flags_to) nflags = 0;
     // the clearing blocks store float2
@@ -1243,7 +1253,7 @@ hipError_t launch_tile_order(uint32_t* ranges, uint32_t num_tiles, uint32_t* ord
     const uint32_t fill_blocks =
         zero_floats ? (uint32_t)std::min<uint64_t>((pairs + ORDER_BLOCK * 4 - 1) / (ORDER_BLOCK * 4) + 1, 2048) : 0u;
     tile_order_kernel<<<8 + fill_blocks, ORDER_BLOCK, 0, s>>>(ranges, num_tiles, order, shrunk_init, fix_empty ? 1 : 0,
-                                                              flags_from, flags_to, nflags, aux_out, zero, zero_floats);
+                                                              flags_from, flags_to, nflags, aux_out, zero, zero_floats, full_start);
     return hipGetLastError();
 }
 

@@ -122,7 +122,7 @@ constexpr uint32_t CUT_BINS = 64;         // depth bins, equal spans of the raw 
 constexpr float CUT_SCALE = 4096.0f;      // fixed-point units per nat of -ln(1 - alpha)
 constexpr uint32_t CUT_FRONT = 16;        // front bins, whose masses every splat adds
 constexpr uint32_t CUT_MAX_BW = 4096;     // tile columns the row kernel holds in LDS
-constexpr uint32_t CUT_AUTO_PER_TILE = 2048;   // VS_CUTOFF_AUTO: listed pairs per tile that turn it on
+constexpr uint32_t CUT_AUTO_PER_TILE = 2048;   // listed pairs per tile that turn it on (VS_CUTOFF_AUTO; hidden when off)
 struct CutArgs {
     uint32_t num_splats, tile_bw, tile_bh;
     const uint32_t* counts;          // [N] tiles per splat (0: not listed anywhere)
@@ -138,6 +138,21 @@ struct CutArgs {
     uint32_t* pend_total;            // the tiles still short of it after the front bins (all rows)
 };
 
+// Per-tile list lengths without the lists (launch_tile_counts).
+constexpr uint32_t TILE_COUNT_SPLATS = 8192;           // most splats of a workgroup: its 16-bit differences cannot overflow
+constexpr uint32_t TILE_COUNT_MAX_LDS = 96u << 10;     // most bytes of a workgroup's difference table
+struct TileCountArgs {
+    uint32_t num_splats, tile_bw, tile_bh;
+    const uint32_t* counts;          // [N] tiles per splat
+    const float4* proj;              // [N][PROJ_Q] projected rows
+    uint32_t* partial;               // [groups][words] the workgroups' packed differences
+    int32_t* diff;                   // [bh][bw + 1] their sum, zeroed by the caller
+    uint32_t* start;                 // [T + 1] out: exclusive scan of the tiles' list lengths
+};
+uint32_t tile_count_words(uint32_t bw, uint32_t bh);      // 32-bit words of one difference table
+uint32_t tile_count_groups(uint32_t num_splats);          // workgroups of the counting pass
+hipError_t launch_tile_counts(const TileCountArgs& a, hipStream_t s);
+
 struct RasterArgs {
     uint32_t img_w, img_h, tile_bw, tile_bh, num_tiles;
     uint32_t num_splats;             // ids at or past it (only a corrupt list holds them) are skipped
@@ -146,7 +161,8 @@ struct RasterArgs {
     const uint32_t* gids;            // sorted intersections -> global splat id
     const uint32_t* ranges;          // [T,2]
     uint32_t* ranges_shrunk;         // [T,2] written by bwd-info passes (may alias nothing else)
-    uint32_t* aux_ranges;            // [T,2] the caller's copy of the shrunk ranges (bwd-info passes), or null
+    uint32_t* aux_ranges;            // [T,2] the caller's copy of the shrunk ranges (bwd-info passes), or null; its
+                                     // starts, set before, may index longer lists than `ranges`
     const float4* proj;              // [N][PROJ_Q] projected rows
     const float4* proj_aux;
     const float4* proj_surf;         // [N][4] surfels (vs_surfel.h layout) or null
@@ -335,11 +351,14 @@ hipError_t launch_tile_ranges(const uint32_t* tiles, uint32_t n, uint32_t num_ti
 // lagged render's pinned readback slot).
 // `aux_out` (optional): the caller's tile offsets, set like `shrunk_init`
 // when that is given (the forward raises their ends too), else to the
-// (fixed) ranges.
+// (fixed) ranges.  `full_start` (optional, [T + 1]): the aux offsets index
+// other lists, of which these are the fronts: tile t's starts at
+// full_start[t] and ends at full_start[t + 1] (an empty one is (0, 0)).
 hipError_t launch_tile_order(uint32_t* ranges, uint32_t num_tiles, uint32_t* order, hipStream_t s,
                              uint32_t* shrunk_init = nullptr, bool fix_empty = false,
                              const uint32_t* flags_from = nullptr, uint32_t* flags_to = nullptr, uint32_t nflags = 0,
-                             uint32_t* aux_out = nullptr, float* zero = nullptr, uint64_t zero_floats = 0);
+                             uint32_t* aux_out = nullptr, float* zero = nullptr, uint64_t zero_floats = 0,
+                             const uint32_t* full_start = nullptr);
 hipError_t launch_ranges_init(uint32_t* ranges, uint32_t num_tiles, hipStream_t s);
 hipError_t launch_tiles_from_ranges(const uint32_t* ranges, uint32_t num_tiles, uint32_t n, uint32_t* tiles,
                                     hipStream_t s);
