@@ -245,19 +245,24 @@ def test_long_lists_with_the_cutoff_off(ctx, n, size, focal, pass_name, mode_nam
     ref = po.render_forward(cam, size, sc.transforms, sc.sh_coeffs, sc.raw_opacities, flags=flags)
     t_count = ((size[0] + 15) // 16) * ((size[1] + 15) // 16)
     assert ref.info.num_intersections >= 2048 * t_count, ref.info.num_intersections / t_count
-    if lagged:
-        va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode).state.free()
-        ctx.set_lagged_counts(True)
+    # a first render at a size counts the full lists' offsets in a walk of their
+    # own, one whose size has a capacity hint in its projection's
+    want = ref.get(po.F_TILE_OFFSETS_SHRUNK if pass_.bwd_info() else po.F_TILE_OFFSETS).reshape(-1, 2)
+    first = va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode)
+    np.testing.assert_array_equal(first.aux.tile_offsets.cpu().numpy().reshape(-1, 2).view(np.uint32), want)
+    if first.state is not None:
+        first.state.free()
+    ctx.set_lagged_counts(lagged)
     out = va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode)
     torch.cuda.synchronize()
     offsets = out.aux.tile_offsets.cpu().numpy().reshape(-1, 2).view(np.uint32)
     if not pass_.bwd_info():
-        np.testing.assert_array_equal(offsets, ref.get(po.F_TILE_OFFSETS).reshape(-1, 2))
+        np.testing.assert_array_equal(offsets, want)
         ctx.set_depth_cutoff(ctx.CUTOFF_ON)
         cut = va.render(cam, size, t, s, o, pass_=pass_, render_mode=mode)
         assert torch.equal(out.out_img, cut.out_img)
         return
-    np.testing.assert_array_equal(offsets, ref.get(po.F_TILE_OFFSETS_SHRUNK).reshape(-1, 2))
+    np.testing.assert_array_equal(offsets, want)
     img = out.out_img.cpu().numpy()
     assert np.array_equal(img.view(np.uint32), ref.get(po.F_OUT_IMG).view(np.uint32))
     np.testing.assert_array_equal(out.aux.visible.cpu().numpy(), ref.get(po.F_VISIBLE))

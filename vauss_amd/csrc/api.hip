@@ -737,6 +737,18 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
         }
     }
 
+    // A hidden cutoff (below) is expected where the size's capacity hint, or the
+    // arena it set, is past its bar: the projection then also tallies the tile
+    // lists' lengths.
+    const uint32_t count_words = tile_count_words(st->tbw, st->tbh);
+    const bool hidden_ok = ctx->depth_cutoff == VS_CUTOFF_OFF && !geometry && !surfel && count_words * 4u <= TILE_COUNT_MAX_LDS;
+    bool tally = false;
+    if (hidden_ok && out->tile_offsets && N > 0 && count_words * 4u <= TALLY_MAX_LDS) {
+        size_t expect = isect_cap;
+        if (!lagged && !ctx->caps.hint(key, N, limit, expect)) expect = 0;
+        tally = expect >= (size_t)CUT_AUTO_PER_TILE * T;
+    }
+
     // ---- per-splat arena -----------------------------------------------------
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += align256(bytes); return o; };
@@ -751,6 +763,7 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
     const size_t o_cnt = take(CNT_COUNT * 4);
     const size_t o_rng = take((size_t)T * 8), o_rngs = take((size_t)T * 8);
     const size_t o_ord = take((size_t)8 * ((T + 7) / 8) * 4);
+    const size_t o_tally = tally ? take((size_t)tally_groups(N) * count_words * 4) : 0;
     VS_HIP(lib_alloc(ctx, &st->arena, off, s), "hipMallocAsync(splat arena)");
     char* base = static_cast<char*>(st->arena);
     st->counts = reinterpret_cast<uint32_t*>(base + o_counts);
@@ -781,6 +794,8 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
         pa.proj_aux = st->proj_aux; pa.proj_surf = st->proj_surf; pa.compact = st->compact; pa.block_stats = st->block_stats;
         pa.visible = bwd_info ? st->visible : nullptr;   // cleared by the projection
         pa.ranges = st->ranges; pa.num_tiles = T;         // initialised by the projection
+        pa.tally = tally ? reinterpret_cast<uint32_t*>(base + o_tally) : nullptr;
+        pa.tally_words = count_words;
         VS_HIP(launch_project(pa, s), "project kernel");
         VS_HIP(launch_finalize_counts(st->block_stats, nblocks, st->counters, isect_cap, s,
                                       lag_slot ? lag_slot->host : nullptr), "projection counts");
@@ -828,9 +843,7 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
     // median channel indexes the lists, keep them.
     const bool tables = !surfel && N > 0 && I > 0 && st->tbw <= CUT_MAX_BW && cut_words * 6u <= (256ull << 20);
     const bool heavy = (uint64_t)I >= (uint64_t)CUT_AUTO_PER_TILE * T;
-    const uint32_t count_words = tables ? tile_count_words(st->tbw, st->tbh) : 0u;
-    const bool hidden = tables && heavy && ctx->depth_cutoff == VS_CUTOFF_OFF && !geometry &&
-                        count_words * 4u <= TILE_COUNT_MAX_LDS;
+    const bool hidden = tables && heavy && hidden_ok;
     const bool cutoff = hidden || (tables && (ctx->depth_cutoff == VS_CUTOFF_ON ||
                                               (ctx->depth_cutoff == VS_CUTOFF_AUTO && heavy)));
     st->hidden = hidden;
@@ -857,7 +870,7 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
         const size_t o_ptot = cutoff ? itake(4) : 0;
         const size_t o_diff = hidden ? itake(((size_t)st->tbw + 1u) * st->tbh * 4) : 0;
         const size_t o_fstart = hidden ? itake(((size_t)T + 1u) * 4) : 0;
-        const size_t o_fpart = hidden ? itake((size_t)tile_count_groups(N) * count_words * 4) : 0;
+        const size_t o_fpart = hidden && !tally ? itake((size_t)tile_count_groups(N) * count_words * 4) : 0;
         // serves both sorts (the depth sort on 9-bit digits, the tile sort on tile_rb-bit ones)
         const uint32_t tile_rb = tile_radix_bits(tile_bits);
         const size_t o_tmp = itake(std::max(sort_tmp_bytes(I, false, tile_rb), sort_tmp_bytes(M, false, DEPTH_RADIX_BITS)));
@@ -917,7 +930,9 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
             StageTimer tm(ctx, ST_EMIT);
             TileCountArgs ta{};
             ta.num_splats = N; ta.tile_bw = st->tbw; ta.tile_bh = st->tbh; ta.counts = st->counts; ta.proj = st->proj;
-            ta.partial = reinterpret_cast<uint32_t*>(ib + o_fpart);
+            ta.partial = reinterpret_cast<uint32_t*>(tally ? base + o_tally : ib + o_fpart);
+            ta.groups = tally ? tally_groups(N) : tile_count_groups(N);
+            ta.tallied = tally ? 1u : 0u;
             ta.diff = reinterpret_cast<int32_t*>(ib + o_diff);
             ta.start = full_start = reinterpret_cast<uint32_t*>(ib + o_fstart);
             VS_HIP(launch_fill_u32(reinterpret_cast<uint32_t*>(ta.diff), 0u, ((uint64_t)st->tbw + 1u) * st->tbh, s),
@@ -1004,6 +1019,7 @@ static vs_status render_forward(vs_ctx* ctx, const vs_camera* cam, const vs_spla
         ra.bg_r = background[0]; ra.bg_g = background[1]; ra.bg_b = background[2];
         ra.gids = st->gids; ra.ranges = st->ranges; ra.ranges_shrunk = st->ranges_shrunk;
         ra.aux_ranges = bwd_info ? out->tile_offsets : nullptr;
+        ra.full_start = full_start;
         ra.proj = st->proj; ra.proj_aux = st->proj_aux;
         // surfels outside training take the median by the surface criterion (gaussian_splats.rs:100-106)
         ra.proj_surf = st->proj_surf; ra.surf_crit = (surfel && pass_surface_criterion(pass)) ? 1u : 0u;

@@ -15,6 +15,7 @@
 // yields each tile's list in (depth bits, global id) order.  Counting and
 // emission test only the tiles near the ellipse's boundary (see walk_rows).
 #include <algorithm>
+#include <type_traits>
 #include "vs_device.h"
 #include "vs_camera.h"
 #include "vs_sh.h"
@@ -566,10 +567,56 @@ VS_DEV F3 load_color(const SHT* __restrict__ sh, uint32_t g, F3 mean, const vs_c
               clampf(finite(b) ? b : 0.0f, -100.0f, 100.0f)};
 }
 
-template <int DEG, int MODEL, bool GEOM, typename SHT>
-__global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(ProjectArgs a) {
+// The wavefront's next ticket (0, 1, 2, ...) from an LDS counter.  Every lane
+// adds 1, which the compiler makes one add of 64; a branch on the lane around
+// one lane's add would let divergent control flow reach the loop around it.
+VS_DEV uint32_t wave_ticket(uint32_t* counter) {
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t k = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return (uint32_t)__builtin_amdgcn_readlane((int)k, 0) / 64u;
+}
+
+// A workgroup's table of tile-list length differences in LDS, two 16-bit
+// entries a word (see tile_count_kernel).
+struct DiffSink {
+    uint32_t* table;      // LDS
+    uint32_t w1;
+    VS_DEV void add(uint32_t i, uint32_t v) const { atomicAdd(&table[i >> 1], (i & 1u) ? v << 16 : v); }
+    VS_DEV void run(uint32_t ty, uint32_t ia, uint32_t ib) const {
+        add(ty * w1 + ia, 1u);
+        add(ty * w1 + ib, 0xFFFFFFFFu);
+    }
+    VS_DEV void tile(uint32_t tx, uint32_t ty) const { run(ty, tx, tx + 1u); }
+};
+
+// TALLY: the counting walk also adds its tiles to a difference table, one per
+// workgroup, which therefore is of TALLY_BLOCK lanes (the table and the walk's
+// arrays leave room for one workgroup per CU) and takes every gridDim.x-th
+// block of splats.  Chosen for views that the size's capacity hint expects to
+// list thousands of pairs a tile: their lists' lengths then need no walk of
+// their own (3M heavy-tailed splats, 2560x1440: the projection 530 -> 640 us,
+// the separate walk's 590 us saved).
+constexpr int TALLY_BLOCK = 1024;
+
+template <int DEG, int MODEL, bool GEOM, typename SHT, bool TALLY>
+__global__ void __launch_bounds__(TALLY ? TALLY_BLOCK : PROJ_BLOCK) project_kernel(ProjectArgs a) {
+    constexpr uint32_t PB = TALLY ? TALLY_BLOCK : PROJ_BLOCK;
     const vs_camera& u = a.cam;
-    const uint32_t g = blockIdx.x * PROJ_BLOCK + threadIdx.x;
+    using Lds = std::conditional_t<TALLY, CountLds, RowLds>;
+    __shared__ Lds s_walk[PB / 64];
+    __shared__ uint32_t s_next;
+    extern __shared__ uint32_t s_diff[];
+    const uint32_t lane = lane_id();
+    Lds& L = s_walk[threadIdx.x / 64];
+    if constexpr (TALLY) {
+        if (threadIdx.x == 0) s_next = 0u;
+        for (uint32_t i = threadIdx.x; i < a.tally_words; i += PB) s_diff[i] = 0u;
+        __syncthreads();
+    }
+    // Splat g on this lane: its row, outputs and tile count (the wavefront's
+    // lanes walk their boxes together).
+    struct Counted { uint32_t hits, dbits; bool visible; };
+    auto project = [&](uint32_t g) -> Counted {
     bool visible = false;
     float px = 0.0f, py = 0.0f, power = 0.0f, radius = 0.0f, opac_out = 0.0f;
     S2 conic{0.0f, 0.0f, 0.0f};
@@ -680,12 +727,13 @@ __global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(ProjectArgs a) {
 
     // Tile counting (kernels/helpers.rs:253-273): the StopThePop test on every
     // tile of the box, in a load-balanced walk over the wavefront's boxes.
-    __shared__ RowLds s_walk[PROJ_BLOCK / 64];
-    const uint32_t lane = lane_id();
-    RowLds& L = s_walk[threadIdx.x / 64];
     uint32_t hits = 0u;
     if (__ballot(visible) != 0ull) {   // a wavefront without a visible splat skips the walk
-        walk_rows<false>(L, visible, bb, px, py, conic, power, 0u, 0u, 0u, a.tile_bw, nullptr, nullptr, 0u);
+        if constexpr (TALLY)
+            walk_rows<false, false>(L, visible, bb, px, py, conic, power, 0u, 0u, 0u, a.tile_bw, nullptr, nullptr, 0u,
+                                    CutFilter{nullptr, nullptr}, 0u, DiffSink{s_diff, a.tile_bw + 1u});
+        else
+            walk_rows<false>(L, visible, bb, px, py, conic, power, 0u, 0u, 0u, a.tile_bw, nullptr, nullptr, 0u);
         hits = L.acc[lane];
     }
 
@@ -697,35 +745,73 @@ __global__ void __launch_bounds__(PROJ_BLOCK) project_kernel(ProjectArgs a) {
         a.compact[g] = visible ? g + 1u : 0u;
         if (a.visible) a.visible[g] = 0.0f;
     }
+    return Counted{hits, dbits, visible};
+    };
+
+    // Statistics per PROJ_BLOCK splats, reduced by finalize_counts_kernel (no
+    // global atomics: a same-address atomic from every wave serialises across
+    // the XCDs).
+    const uint32_t nb = (a.num_splats + PROJ_BLOCK - 1u) / PROJ_BLOCK;
+    auto put_stats = [&](uint32_t at, uint32_t sum, uint32_t vis, uint32_t mn, uint32_t mxm, uint32_t emit) {
+        a.block_stats[BS_HITS * nb + at] = sum;
+        a.block_stats[BS_VISIBLE * nb + at] = vis;
+        a.block_stats[BS_DMIN * nb + at] = mn;
+        a.block_stats[BS_DMAX * nb + at] = mxm;
+        a.block_stats[BS_EMIT * nb + at] = emit;
+    };
     // every tile's range starts as (0xFFFFFFFF, 0): the tile sort's range pass
     // lowers starts and raises ends
-    for (uint32_t t = g; t < a.num_tiles; t += gridDim.x * PROJ_BLOCK)
-        reinterpret_cast<uint2*>(a.ranges)[t] = make_uint2(0xFFFFFFFFu, 0u);
-
-    // Block statistics, reduced by finalize_counts_kernel (no global atomics:
-    // a same-address atomic from every wave serialises across the XCDs).
-    __shared__ uint32_t s_sum[PROJ_BLOCK / 64], s_vis[PROJ_BLOCK / 64], s_min[PROJ_BLOCK / 64], s_max[PROJ_BLOCK / 64];
-    __shared__ uint32_t s_emit[PROJ_BLOCK / 64];
-    const uint32_t wsum = wave_sum(hits);
-    const uint32_t wvis = (uint32_t)__popcll(__ballot(visible));
-    const uint32_t wemit = (uint32_t)__popcll(__ballot(hits > 0u));
-    const uint32_t wmin = wave_min(visible ? dbits : 0xFFFFFFFFu);
-    const uint32_t wmax = wave_max(visible ? dbits : 0u);
-    const uint32_t wave = threadIdx.x / 64;
-    if (lane == 0) { s_sum[wave] = wsum; s_vis[wave] = wvis; s_min[wave] = wmin; s_max[wave] = wmax; s_emit[wave] = wemit; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t bs = 0, bv = 0, bmn = 0xFFFFFFFFu, bmx = 0u, be = 0;
+    auto init_ranges = [&]() {
+        for (uint32_t t = blockIdx.x * PB + threadIdx.x; t < a.num_tiles; t += gridDim.x * PB)
+            reinterpret_cast<uint2*>(a.ranges)[t] = make_uint2(0xFFFFFFFFu, 0u);
+    };
+    if constexpr (!TALLY) {
+        __shared__ uint32_t s_sum[PB / 64], s_vis[PB / 64], s_min[PB / 64], s_max[PB / 64], s_emit[PB / 64];
+        const Counted c = project(blockIdx.x * PB + threadIdx.x);
+        init_ranges();
+        const uint32_t wsum = wave_sum(c.hits);
+        const uint32_t wvis = (uint32_t)__popcll(__ballot(c.visible));
+        const uint32_t wemit = (uint32_t)__popcll(__ballot(c.hits > 0u));
+        const uint32_t wmin = wave_min(c.visible ? c.dbits : 0xFFFFFFFFu);
+        const uint32_t wmax = wave_max(c.visible ? c.dbits : 0u);
+        const uint32_t wave = threadIdx.x / 64;
+        if (lane == 0) { s_sum[wave] = wsum; s_vis[wave] = wvis; s_min[wave] = wmin; s_max[wave] = wmax; s_emit[wave] = wemit; }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t bs = 0, bv = 0, bmn = 0xFFFFFFFFu, bmx = 0u, be = 0;
 #pragma unroll
-        for (int w = 0; w < PROJ_BLOCK / 64; ++w) {
-            bs += s_sum[w]; bv += s_vis[w]; bmn = min(bmn, s_min[w]); bmx = max(bmx, s_max[w]); be += s_emit[w];
+            for (int w = 0; w < PROJ_BLOCK / 64; ++w) {
+                bs += s_sum[w]; bv += s_vis[w]; bmn = min(bmn, s_min[w]); bmx = max(bmx, s_max[w]); be += s_emit[w];
+            }
+            put_stats(blockIdx.x, bs, bv, bmn, bmx, be);
         }
-        const uint32_t nb = gridDim.x;
-        a.block_stats[BS_HITS * nb + blockIdx.x] = bs;
-        a.block_stats[BS_VISIBLE * nb + blockIdx.x] = bv;
-        a.block_stats[BS_DMIN * nb + blockIdx.x] = bmn;
-        a.block_stats[BS_DMAX * nb + blockIdx.x] = bmx;
-        a.block_stats[BS_EMIT * nb + blockIdx.x] = be;
+    } else {
+        init_ranges();
+        // each wavefront takes the workgroup's next block of PROJ_BLOCK splats
+        // as it gets free: walks differ in length by tens of times
+        for (;;) {
+            const uint32_t blk = blockIdx.x + wave_ticket(&s_next) * gridDim.x;
+            if (blk >= nb) break;
+            uint32_t sum = 0u, vis = 0u, mn = 0xFFFFFFFFu, mxm = 0u, emit = 0u;
+            for (uint32_t i = 0; i < PROJ_BLOCK; i += 64u) {
+                const Counted c = project(blk * PROJ_BLOCK + i + lane);
+                sum += c.hits;
+                vis += (uint32_t)__popcll(__ballot(c.visible));
+                emit += (uint32_t)__popcll(__ballot(c.hits > 0u));
+                mn = min(mn, c.visible ? c.dbits : 0xFFFFFFFFu);
+                mxm = max(mxm, c.visible ? c.dbits : 0u);
+            }
+            sum = wave_sum(sum);
+            mn = wave_min(mn);
+            mxm = wave_max(mxm);
+            // every lane stores the same words: a branch on the lane here ends the
+            // loop body divergent, and the compiler then let the other lanes
+            // start the next turn without lane 0, whose ticket they read
+            put_stats(blk, sum, vis, mn, mxm, emit);
+        }
+        __syncthreads();
+        uint32_t* out = a.tally + (size_t)blockIdx.x * a.tally_words;
+        for (uint32_t i = threadIdx.x; i < a.tally_words; i += PB) out[i] = s_diff[i];
     }
 }
 
@@ -1133,28 +1219,22 @@ __global__ void __launch_bounds__(PROJ_BLOCK) count_kept_kernel(EmitArgs a) {
 // each), because the updates are many and land on few words: 6.7e7 of them
 // into 14,490 entries at 3M heavy-tailed splats and 2560x1440, where global
 // atomics ran at about 25 per ns.  Bound by the walk's chords, as the
-// projection's is.  It takes 0.70 ms there and spares emitting and sorting
-// 3.6e8 pairs (5.3 ms; the training view 6.68 -> 2.48 ms).
+// projection's is.  It takes 0.59 ms there and spares emitting and sorting
+// 3.6e8 pairs (5.3 ms; the training view 6.68 -> 2.4 ms; 1.9 with the lengths
+// tallied in the projection, see TALLY).
 constexpr int TCOUNT_BLOCK = 512;
-struct DiffSink {
-    uint32_t* table;      // LDS
-    uint32_t w1;
-    VS_DEV void add(uint32_t i, uint32_t v) const { atomicAdd(&table[i >> 1], (i & 1u) ? v << 16 : v); }
-    VS_DEV void run(uint32_t ty, uint32_t ia, uint32_t ib) const {
-        add(ty * w1 + ia, 1u);
-        add(ty * w1 + ib, 0xFFFFFFFFu);
-    }
-    VS_DEV void tile(uint32_t tx, uint32_t ty) const { run(ty, tx, tx + 1u); }
-};
-
 __global__ void __launch_bounds__(TCOUNT_BLOCK) tile_count_kernel(TileCountArgs a, uint32_t words, uint32_t per) {
     extern __shared__ uint32_t s_diff[];
     __shared__ CountLds s_walk[TCOUNT_BLOCK / 64];
+    __shared__ uint32_t s_next;
     CountLds& L = s_walk[threadIdx.x / 64];
+    if (threadIdx.x == 0) s_next = 0u;
     for (uint32_t i = threadIdx.x; i < words; i += TCOUNT_BLOCK) s_diff[i] = 0u;
     __syncthreads();
     const uint32_t first = blockIdx.x * per, last = (uint32_t)min((uint64_t)first + per, (uint64_t)a.num_splats);
-    for (uint32_t g0 = first + (threadIdx.x & ~63u); g0 < last; g0 += TCOUNT_BLOCK) {     // uniform per wavefront
+    for (;;) {      // each wavefront takes the next 64 splats as it gets free
+        const uint32_t g0 = first + 64u * wave_ticket(&s_next);
+        if (g0 >= last) break;
         const uint32_t g = g0 + lane_id();
         const bool has = g < last && a.counts[g] > 0u;
         if (__ballot(has) == 0ull) continue;
@@ -1305,27 +1385,40 @@ hipError_t launch_finalize_counts(uint32_t* block_stats, uint32_t nblocks, uint3
     return hipGetLastError();
 }
 
+// Workgroups of a tallying projection: one per CU, or as many as keep a
+// workgroup's splats under 2^15 (its 16-bit entries count splats).
+uint32_t tally_groups(uint32_t n) {
+    const uint32_t blocks = (n + PROJ_BLOCK - 1u) / PROJ_BLOCK;
+    return std::max(std::min(blocks, 256u), (blocks + 126u) / 127u);
+}
 template <int DEG, int MODEL, typename SHT>
-static void launch_project_geom(const ProjectArgs& a, dim3 grid, hipStream_t s, bool geom) {
-    if (geom) project_kernel<DEG, MODEL, true, SHT><<<grid, PROJ_BLOCK, 0, s>>>(a);
-    else project_kernel<DEG, MODEL, false, SHT><<<grid, PROJ_BLOCK, 0, s>>>(a);
+static hipError_t launch_project_geom(const ProjectArgs& a, dim3 grid, hipStream_t s, bool geom) {
+    if (geom) project_kernel<DEG, MODEL, true, SHT, false><<<grid, PROJ_BLOCK, 0, s>>>(a);
+    else if constexpr (MODEL != SURFEL_MODEL) {
+        if (a.tally) {
+            const auto k = project_kernel<DEG, MODEL, false, SHT, true>;
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               (int)TALLY_MAX_LDS);
+            if (e != hipSuccess) return e;
+            k<<<tally_groups(a.num_splats), TALLY_BLOCK, a.tally_words * 4u, s>>>(a);
+        } else project_kernel<DEG, MODEL, false, SHT, false><<<grid, PROJ_BLOCK, 0, s>>>(a);
+    } else project_kernel<DEG, MODEL, false, SHT, false><<<grid, PROJ_BLOCK, 0, s>>>(a);
+    return hipGetLastError();
 }
 template <int DEG, int MODEL>
-static void launch_project_type(const ProjectArgs& a, dim3 grid, hipStream_t s, bool geom) {
-    if (a.sh_half) launch_project_geom<DEG, MODEL, uint16_t>(a, grid, s, geom);
-    else launch_project_geom<DEG, MODEL, float>(a, grid, s, geom);
+static hipError_t launch_project_type(const ProjectArgs& a, dim3 grid, hipStream_t s, bool geom) {
+    return a.sh_half ? launch_project_geom<DEG, MODEL, uint16_t>(a, grid, s, geom)
+                     : launch_project_geom<DEG, MODEL, float>(a, grid, s, geom);
 }
 template <int DEG>
-static void launch_project_model(const ProjectArgs& a, dim3 grid, hipStream_t s, bool geom) {
-    if (a.proj_surf) {                       // surfels: pinhole camera, no gaussian geometry normal
-        launch_project_type<DEG, SURFEL_MODEL>(a, grid, s, false);
-        return;
-    }
+static hipError_t launch_project_model(const ProjectArgs& a, dim3 grid, hipStream_t s, bool geom) {
+    // surfels: pinhole camera, no gaussian geometry normal
+    if (a.proj_surf) return launch_project_type<DEG, SURFEL_MODEL>(a, grid, s, false);
     switch (a.cam.model) {
-    case VS_CAMERA_KB4: launch_project_type<DEG, VS_CAMERA_KB4>(a, grid, s, geom); break;
-    case VS_CAMERA_RT8: launch_project_type<DEG, VS_CAMERA_RT8>(a, grid, s, geom); break;
-    case VS_CAMERA_TPF: launch_project_type<DEG, VS_CAMERA_TPF>(a, grid, s, geom); break;
-    default: launch_project_type<DEG, VS_CAMERA_PINHOLE>(a, grid, s, geom); break;
+    case VS_CAMERA_KB4: return launch_project_type<DEG, VS_CAMERA_KB4>(a, grid, s, geom);
+    case VS_CAMERA_RT8: return launch_project_type<DEG, VS_CAMERA_RT8>(a, grid, s, geom);
+    case VS_CAMERA_TPF: return launch_project_type<DEG, VS_CAMERA_TPF>(a, grid, s, geom);
+    default: return launch_project_type<DEG, VS_CAMERA_PINHOLE>(a, grid, s, geom);
     }
 }
 
@@ -1333,18 +1426,15 @@ hipError_t launch_project(const ProjectArgs& a, hipStream_t s) {
     if (a.num_splats == 0) return hipSuccess;
     const dim3 grid((a.num_splats + PROJ_BLOCK - 1) / PROJ_BLOCK);
     const bool geom = a.proj_aux != nullptr;
-    if (a.decoder) {
-        launch_project_model<NEURAL_DEG>(a, grid, s, geom);
-        return hipGetLastError();
-    }
+    if (a.tally && (geom || a.proj_surf || a.tally_words * 4u > TALLY_MAX_LDS)) return hipErrorInvalidValue;
+    if (a.decoder) return launch_project_model<NEURAL_DEG>(a, grid, s, geom);
     switch (a.sh_degree) {
-    case 0: launch_project_model<0>(a, grid, s, geom); break;
-    case 1: launch_project_model<1>(a, grid, s, geom); break;
-    case 2: launch_project_model<2>(a, grid, s, geom); break;
-    case 3: launch_project_model<3>(a, grid, s, geom); break;
-    default: launch_project_model<4>(a, grid, s, geom); break;
+    case 0: return launch_project_model<0>(a, grid, s, geom);
+    case 1: return launch_project_model<1>(a, grid, s, geom);
+    case 2: return launch_project_model<2>(a, grid, s, geom);
+    case 3: return launch_project_model<3>(a, grid, s, geom);
+    default: return launch_project_model<4>(a, grid, s, geom);
     }
-    return hipGetLastError();
 }
 
 hipError_t launch_compact(const CompactArgs& a, hipStream_t s) {
@@ -1396,18 +1486,21 @@ static uint32_t tile_count_per(uint32_t n) {
 }
 uint32_t tile_count_groups(uint32_t n) { return n ? (n + tile_count_per(n) - 1u) / tile_count_per(n) : 0u; }
 hipError_t launch_tile_counts(const TileCountArgs& a, hipStream_t s) {
-    const uint32_t words = tile_count_words(a.tile_bw, a.tile_bh), groups = tile_count_groups(a.num_splats);
-    const uint32_t entries = (a.tile_bw + 1u) * a.tile_bh, lds = words * 4u;
-    if (!groups || !a.partial || !a.diff || !a.start || lds > TILE_COUNT_MAX_LDS) return hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_count_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)TILE_COUNT_MAX_LDS);
-    if (e != hipSuccess) return e;
-    tile_count_kernel<<<groups, TCOUNT_BLOCK, lds, s>>>(a, words, tile_count_per(a.num_splats));
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    tile_count_sum_kernel<<<dim3((words + TSUM_BLOCK - 1) / TSUM_BLOCK, std::min(groups, TCOUNT_SLICES)), TSUM_BLOCK, 0, s>>>(
-        a.partial, groups, words, entries, a.diff);
-    e = hipGetLastError();
+    const uint32_t words = tile_count_words(a.tile_bw, a.tile_bh);
+    const uint32_t entries = (a.tile_bw + 1u) * a.tile_bh;
+    if (!a.groups || !a.partial || !a.diff || !a.start || words * 4u > TILE_COUNT_MAX_LDS) return hipErrorInvalidValue;
+    if (!a.tallied) {
+        if (a.groups != tile_count_groups(a.num_splats)) return hipErrorInvalidValue;
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(tile_count_kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)TILE_COUNT_MAX_LDS);
+        if (e != hipSuccess) return e;
+        tile_count_kernel<<<a.groups, TCOUNT_BLOCK, words * 4u, s>>>(a, words, tile_count_per(a.num_splats));
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    tile_count_sum_kernel<<<dim3((words + TSUM_BLOCK - 1) / TSUM_BLOCK, std::min(a.groups, TCOUNT_SLICES)), TSUM_BLOCK, 0, s>>>(
+        a.partial, a.groups, words, entries, a.diff);
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // the row totals take the first table's place once the tables are summed
     tile_start_kernel<<<1, TSTART_BLOCK, 0, s>>>(a.diff, a.tile_bw, a.tile_bh, a.partial, a.start);

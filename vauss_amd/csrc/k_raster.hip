@@ -631,7 +631,7 @@ __global__ void __launch_bounds__(FWD_BATCH) raster_fwd_kernel(RasterArgs a) {
             atomicMax(&a.ranges_shrunk[tile * 2 + 1], last);
             // the caller's range ends as far past its own start, which indexes
             // the full list where `ranges` holds its front alone
-            if (a.aux_ranges) atomicMax(&a.aux_ranges[tile * 2 + 1], a.aux_ranges[tile * 2] + (last - lo));
+            if (a.aux_ranges) atomicMax(&a.aux_ranges[tile * 2 + 1], a.full_start ? a.full_start[tile] + (last - lo) : last);
         }
     }
 }

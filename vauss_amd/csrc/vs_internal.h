@@ -69,7 +69,11 @@ struct ProjectArgs {
     float* visible;             // [N] cleared to 0 (the forward marks the splats it blends), or null
     uint32_t* ranges;           // [num_tiles, 2] set to (0xFFFFFFFF, 0) for the tile sort's range pass
     uint32_t num_tiles;
+    uint32_t* tally;            // [tally_groups][tally_words] per-workgroup differences of the tile lists' lengths, or null
+    uint32_t tally_words;       // tile_count_words
 };
+constexpr uint32_t TALLY_MAX_LDS = 72u << 10;          // most bytes of a tallying projection's table (its walk takes 86 KB)
+uint32_t tally_groups(uint32_t num_splats);            // workgroups of a tallying projection
 
 struct CompactArgs {
     uint32_t num_splats;
@@ -146,6 +150,8 @@ struct TileCountArgs {
     const uint32_t* counts;          // [N] tiles per splat
     const float4* proj;              // [N][PROJ_Q] projected rows
     uint32_t* partial;               // [groups][words] the workgroups' packed differences
+    uint32_t groups;                 // tile_count_groups, or tally_groups when the projection filled `partial`
+    uint32_t tallied;
     int32_t* diff;                   // [bh][bw + 1] their sum, zeroed by the caller
     uint32_t* start;                 // [T + 1] out: exclusive scan of the tiles' list lengths
 };
@@ -161,8 +167,8 @@ struct RasterArgs {
     const uint32_t* gids;            // sorted intersections -> global splat id
     const uint32_t* ranges;          // [T,2]
     uint32_t* ranges_shrunk;         // [T,2] written by bwd-info passes (may alias nothing else)
-    uint32_t* aux_ranges;            // [T,2] the caller's copy of the shrunk ranges (bwd-info passes), or null; its
-                                     // starts, set before, may index longer lists than `ranges`
+    uint32_t* aux_ranges;            // [T,2] the caller's copy of the shrunk ranges (bwd-info passes), or null
+    const uint32_t* full_start;      // [T + 1] where the lists they index start, when those are not `ranges`' (or null)
     const float4* proj;              // [N][PROJ_Q] projected rows
     const float4* proj_aux;
     const float4* proj_surf;         // [N][4] surfels (vs_surfel.h layout) or null
