@@ -200,3 +200,20 @@ def test_exact_render_reports_a_sort_give_up():
         ctx.set_sort_spin_limit(None)
     out = va.render(wl.cameras[0], wl.img_size, t, s, o, pass_=va.RasterPass.FLOAT)
     assert out.aux.num_intersections > 500_000
+
+
+# One-sweep look-back over groups of 32 tiles (4096 pairs each up to 2^21 pairs,
+# 8192 above): lengths at a group's edge, one pair past it and inside the next
+# group's last tile; digits
+# from one value to all of them.
+@pytest.mark.parametrize("n", [32 * 4096 - 1, 32 * 4096, 32 * 4096 + 1, 64 * 4096 - 7, 5 * 32 * 4096 + 3 * 4096 + 1,
+                               13 * 32 * 8192 - 1, 13 * 32 * 8192 + 1])
+@pytest.mark.parametrize("span", [1, 300, 2 ** 32])
+def test_sort_group_edges(n, span):
+    rng = np.random.default_rng(n % 1000 + span % 7)
+    keys = rng.integers(0, span, n, dtype=np.uint64).astype(np.uint32)
+    vals = np.arange(n, dtype=np.uint32)
+    gk, gv = _sort(keys, vals, 32, 0)
+    ek, ev = _expected(keys, vals, 32, 0)
+    np.testing.assert_array_equal(gk, ek)
+    np.testing.assert_array_equal(gv, ev)

@@ -10,7 +10,8 @@
 //  * one-sweep (n >= ONESWEEP_MIN): one histogram kernel counts the digits of
 //    every pass in a single read of the keys; each pass is then a single
 //    kernel in which each block publishes its tile's per-digit counts and sums
-//    its predecessors' counts by decoupled look-back (a block only waits on
+//    its predecessors' counts by decoupled look-back, over its own group of
+//    tiles and then over whole groups (a block only waits on
 //    lower-indexed blocks, which are dispatched first and publish before they
 //    wait, so the chain drains; a bounded spin turns anything else into a
 //    reported error, not a hang);
@@ -20,6 +21,7 @@
 //
 // Ranking in (wave, step, lane) order with waves owning consecutive key
 // ranges keeps every pass stable, so the sort is stable.
+#include <type_traits>
 #include "vs_internal.h"
 
 namespace vs {
@@ -87,63 +89,93 @@ __global__ void __launch_bounds__(SORT_BLOCK) sort_upsweep_kernel(const K* __res
     table[(size_t)d * nblocks + blockIdx.x] = c;
 }
 
-// Block-level ranking of one tile of up to BLOCK * ITEMS keys, in two
-// phases so that a one-sweep pass can publish its digit counts (and look back)
-// between them:
-//  * count(): loads the tile, ranks every key among the equal digits of its
-//    wavefront (ballot matching), and turns the per-wave digit histograms into
-//    each wave's exclusive offset within its digit; returns, in thread
-//    d < 2^RB, the tile's count of digit d;
-//  * place(): from those counts, digit_start[d] (the first LDS slot of digit d)
-//    and the digit-ordered (stable) tile in s_keys / s_vals.
+// n words at p as a buffer: stores take a 32-bit byte offset, and one past the
+// end (a bad rank, or a slot past the tile's keys) is dropped.  n < 2^30.
+using WordBuf = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ WordBuf word_buf(uint32_t* p, uint32_t n) {
+    return __builtin_amdgcn_make_buffer_rsrc(p, 0, n * 4u, 0x00027000);
+}
+__device__ __forceinline__ void word_put(WordBuf b, uint32_t at, uint32_t v) {
+    __builtin_amdgcn_raw_buffer_store_b32(v, b, at < (1u << 30) ? at * 4u : 0xFFFFFFF0u, 0, 0);
+}
+
+// Block-level ranking of one tile of BLOCK * ITEMS keys:
+//  * load(): the tile, in (wave, step, lane) order; keys past the end are all
+//    ones, so they rank behind every key of the tile and need no test;
+//  * count(): ranks every key among the equal digits of its wavefront (ballot
+//    matching) and turns the per-wave digit histograms into each wave's
+//    exclusive offset within its digit; returns, in thread d < 2^RB, the tile's
+//    count of digit d, for a one-sweep pass to publish (and look back) before
+//  * starts(): digit_start[d] (the tile's first slot of digit d) and pos[],
+//    each key's slot in the stable digit order.
+// The tile is then reordered through one LDS buffer, the keys first and the
+// values after them.  A pass over a long input lasts as long as its tiles'
+// serial steps (load, rank, look back, scatter) overlap across the two
+// workgroups that a CU's registers hold (117 VGPRs of 4 waves per SIMD; 6 or 5
+// spill and cost twice the time), so it is the instructions per key that
+// count: no bounds tests, three-input logic for the matching, mbcnt for the
+// rank.  With the grouped look-back below, sorts of random pairs on 32 bits:
+// 30M 855 -> 801 us, 8M 256 -> 220, 3M 149 -> 129 (on 14 bits 88 -> 76).
 template <typename K, int BLOCK, int ITEMS, int RB = 8>
 struct TileRanker {
     static constexpr uint32_t R = 1u << RB;   // digits
+    static constexpr uint32_t TILE = BLOCK * ITEMS;
     static_assert(BLOCK >= (int)R && BLOCK % 64 == 0, "one thread per digit");
+    static_assert(TILE <= 1u << 16, "ranks are kept in 16 bits");
     static constexpr int WAVES = BLOCK / 64;
     K key[ITEMS];
-    uint32_t val[ITEMS], dig[ITEMS], rank[ITEMS];
+    uint32_t val[ITEMS], pos[ITEMS];
     uint32_t run = 0;
 
-    __device__ __forceinline__ uint32_t count(const K* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
-                                              uint32_t base, uint32_t n, uint32_t shift, uint32_t (*wave_hist)[R]) {
+    // Issues every load of the tile before any ranking step, so a wavefront
+    // waits for memory once rather than once per step.
+    __device__ __forceinline__ void load(const K* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, uint32_t base,
+                                         uint32_t n) {
         const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        // Issue every load of the tile before any ranking step, so a wavefront
-        // waits for memory once rather than once per step.
-        const uint32_t wbase = base + wave * (64 * ITEMS);
+        const uint32_t first = wave * (64 * ITEMS) + lane;
+        const uint32_t left = min(n - base, TILE);
+        if constexpr (sizeof(K) == 4) {
+            // one lane offset and constant ones; past the end reads 0
+            const WordBuf kb = word_buf(const_cast<K*>(keys_in) + base, left), vb = word_buf(const_cast<uint32_t*>(vals_in) + base, left);
 #pragma unroll
-        for (int s = 0; s < ITEMS; ++s) {
-            const uint32_t idx = wbase + s * 64 + lane;
-            key[s] = idx < n ? keys_in[idx] : (K)0;
-        }
+            for (int s = 0; s < ITEMS; ++s) key[s] = __builtin_amdgcn_raw_buffer_load_b32(kb, first * 4u + s * 256u, 0, 0);
 #pragma unroll
-        for (int s = 0; s < ITEMS; ++s) {
-            const uint32_t idx = wbase + s * 64 + lane;
-            val[s] = idx < n ? vals_in[idx] : 0u;
+            for (int s = 0; s < ITEMS; ++s) val[s] = __builtin_amdgcn_raw_buffer_load_b32(vb, first * 4u + s * 256u, 0, 0);
+            if (left < TILE) {       // uniform
+#pragma unroll
+                for (int s = 0; s < ITEMS; ++s)
+                    if (first + s * 64 >= left) key[s] = 0xFFFFFFFFu;
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < ITEMS; ++s) key[s] = first + s * 64 < left ? keys_in[base + first + s * 64] : (K)~(K)0;
+#pragma unroll
+            for (int s = 0; s < ITEMS; ++s) val[s] = first + s * 64 < left ? vals_in[base + first + s * 64] : 0u;
         }
+    }
+
+    __device__ __forceinline__ uint32_t count(uint32_t base, uint32_t n, uint32_t shift, uint32_t (*wave_hist)[R]) {
+        const uint32_t wave = threadIdx.x >> 6;
         for (uint32_t i = threadIdx.x; i < WAVES * R; i += BLOCK) (&wave_hist[0][0])[i] = 0;
         __syncthreads();
-
-        const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
         for (int s = 0; s < ITEMS; ++s) {
-            const uint32_t idx = wbase + s * 64 + lane;
-            const bool valid = idx < n;
             const uint32_t d = digit_rb<RB>(key[s], shift);
-            dig[s] = valid ? d : R;
-            uint64_t peers = __ballot(valid);
+            // the lanes with this lane's digit: per bit, keep those whose bit
+            // equals this lane's (m: the bit spread over a word)
+            uint32_t lo = 0xFFFFFFFFu, hi = 0xFFFFFFFFu;
 #pragma unroll
             for (int b = 0; b < RB; ++b) {
-                const uint64_t bal = __ballot((d >> b) & 1u);
-                peers &= ((d >> b) & 1u) ? bal : ~bal;
+                const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)d, (uint32_t)b, 1u);
+                const uint64_t bal = __ballot(m != 0u);
+                lo = __builtin_amdgcn_bitop3_b32(lo, (uint32_t)bal, m, 0x90);           // lo & ~(bal ^ m)
+                hi = __builtin_amdgcn_bitop3_b32(hi, (uint32_t)(bal >> 32), m, 0x90);
             }
-            uint32_t r = 0;
-            if (valid) {
-                const uint32_t before = wave_hist[wave][d];
-                r = before + (uint32_t)__popcll(peers & lt_mask);
-                if ((peers & lt_mask) == 0) wave_hist[wave][d] = before + (uint32_t)__popcll(peers);
-            }
-            rank[s] = r;
+            const uint32_t before = wave_hist[wave][d];
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+            pos[s] = before + below;
+            // every lane of a digit stores the same total
+            wave_hist[wave][d] = before + (uint32_t)(__popc(lo) + __popc(hi));
             __builtin_amdgcn_wave_barrier();
         }
         __syncthreads();
@@ -157,12 +189,13 @@ struct TileRanker {
                 wave_hist[w][d] = run;
                 run += c;
             }
+            // the keys past the end, last of the highest digit
+            if (d == digit_rb<RB>((K)~(K)0, shift) && n - base < TILE) run -= TILE - (n - base);
         }
         return run;
     }
 
-    __device__ __forceinline__ void place(uint32_t (*wave_hist)[R], uint32_t* digit_start, uint32_t* s_tot,
-                                          K* s_keys, uint32_t* s_vals) {
+    __device__ __forceinline__ void starts(uint32_t shift, uint32_t (*wave_hist)[R], uint32_t* digit_start, uint32_t* s_tot) {
         const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const uint32_t d = threadIdx.x;
         // exclusive scan of the digit counts over the R digits
@@ -179,18 +212,46 @@ struct TileRanker {
         if (d < R) {
             uint32_t wo = 0;
             for (uint32_t w = 0; w < wave; ++w) wo += s_tot[w];
-            digit_start[d] = wo + incl - run;
+            const uint32_t start = wo + incl - run;
+            digit_start[d] = start;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) wave_hist[w][d] += start;
         }
+        __syncthreads();
+        // the digits are formed again: kept from count(), with their addresses,
+        // they took 16 registers through the look-back
+#pragma unroll
+        for (int s = 0; s < ITEMS; ++s) asm volatile("" : "+v"(key[s]));
+#pragma unroll
+        for (int s = 0; s < ITEMS; ++s) pos[s] += wave_hist[wave][digit_rb<RB>(key[s], shift)];
+    }
+
+    // The tile in digit order through `buf`: visit(i, key) for each slot i below
+    // `count` returns where the pair goes and put_val(to, value) stores its
+    // value there.  Four slots' addresses are live at a time: all of them at
+    // once took registers that cost a workgroup per CU.
+    template <typename Visit, typename Put>
+    __device__ __forceinline__ void scatter(K* buf, uint32_t count, Visit&& visit, Put&& put_val) {
+        uint32_t to[ITEMS];
+#pragma unroll
+        for (int s = 0; s < ITEMS; ++s) buf[pos[s]] = key[s];
         __syncthreads();
 #pragma unroll
-        for (int s = 0; s < ITEMS; ++s) {
-            if (dig[s] < R) {
-                const uint32_t pos = digit_start[dig[s]] + wave_hist[wave][dig[s]] + rank[s];
-                s_keys[pos] = key[s];
-                s_vals[pos] = val[s];
-            }
+        for (int j = 0; j < ITEMS; ++j) {
+            const uint32_t i = threadIdx.x + (uint32_t)j * BLOCK;
+            to[j] = i < count ? visit(i, buf[i]) : 0xFFFFFFFFu;
+            if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
+        uint32_t* vbuf = reinterpret_cast<uint32_t*>(buf);
+#pragma unroll
+        for (int s = 0; s < ITEMS; ++s) vbuf[pos[s]] = val[s];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; ++j) {
+            put_val(to[j], vbuf[threadIdx.x + (uint32_t)j * BLOCK]);
+            if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
     }
 };
 
@@ -202,31 +263,22 @@ __global__ void __launch_bounds__(SORT_BLOCK) sort_scatter_kernel(const K* __res
     __shared__ uint32_t wave_hist[SORT_WAVES][256];
     __shared__ uint32_t digit_start[256];
     __shared__ uint32_t s_tot[SORT_WAVES];
-    __shared__ K s_keys[SORT_TILE];
-    __shared__ uint32_t s_vals[SORT_TILE];
-
-    __shared__ uint32_t s_gstart[256];
+    __shared__ uint32_t s_off[256];         // digit d's first global slot less its first tile slot
+    __shared__ K s_buf[SORT_TILE];
 
     const uint32_t n = n_dev ? min(*n_dev, n_cap) : n_cap;
     const uint32_t base = blockIdx.x * SORT_TILE;
     if (base >= n) return;   // uniform per block
-    {
-        TileRanker<K, SORT_BLOCK, SORT_ITEMS> rk;
-        rk.count(keys_in, vals_in, base, n, shift, wave_hist);
-        rk.place(wave_hist, digit_start, s_tot, s_keys, s_vals);
-    }
-    if (threadIdx.x < 256) s_gstart[threadIdx.x] = offsets[(size_t)threadIdx.x * nblocks + blockIdx.x];
-    __syncthreads();
-    const uint32_t count = min(SORT_TILE, n - base);
-    for (uint32_t i = threadIdx.x; i < count; i += SORT_BLOCK) {
-        const K k = s_keys[i];
-        const uint32_t d = digit_of(k, shift);
-        const uint32_t gpos = s_gstart[d] + (i - digit_start[d]);
-        if (gpos < n) {   // always true for a consistent table; keeps a bad rank from writing out of bounds
-            keys_out[gpos] = k;
-            vals_out[gpos] = s_vals[i];
-        }
-    }
+    TileRanker<K, SORT_BLOCK, SORT_ITEMS> rk;
+    rk.load(keys_in, vals_in, base, n);
+    rk.count(base, n, shift, wave_hist);
+    rk.starts(shift, wave_hist, digit_start, s_tot);
+    if (threadIdx.x < 256) s_off[threadIdx.x] = offsets[(size_t)threadIdx.x * nblocks + blockIdx.x] - digit_start[threadIdx.x];
+    rk.scatter(s_buf, min(SORT_TILE, n - base), [&](uint32_t i, K k) {
+        const uint32_t gpos = s_off[digit_of(k, shift)] + i;
+        if (gpos < n) keys_out[gpos] = k;   // always true for a consistent table; keeps a bad rank from writing out of bounds
+        return gpos;
+    }, [&](uint32_t to, uint32_t v) { if (to < n) vals_out[to] = v; });
 }
 
 // ---- one-sweep schedule ---------------------------------------------------------
@@ -272,6 +324,19 @@ constexpr uint32_t OS_AGGREGATE = 1u << 30;            // status: this tile's ow
 constexpr uint32_t OS_PREFIX = 2u << 30;               // status: count of this tile and all before it
 constexpr uint32_t OS_VALUE = (1u << 30) - 1u;
 constexpr int LOOKBACK = VS_LOOKBACK;                  // predecessor statuses read per look-back step
+// Tiles in groups: every tile also adds its digit counts to its group's (an
+// arrival count above OS_GROUP_SHIFT beside the sum), and a group's last tile
+// publishes the group's prefix, so a look-back reads at most its own group's
+// tiles and then whole groups: with about 500 tiles in flight one read tile by
+// tile takes up to 64 dependent steps of 8 tiles, by groups up to 4 + 4.
+constexpr uint32_t OS_GROUP = 32;
+constexpr uint32_t OS_GROUP_SHIFT = 24;
+constexpr uint32_t OS_GROUP_SUM = (1u << OS_GROUP_SHIFT) - 1u;
+static_assert(OS_GROUP * OS_TILE <= OS_GROUP_SUM && OS_GROUP * OS_SMALL_TILE <= OS_GROUP_SUM, "a group's count fits below its arrivals");
+constexpr int GROUP_LOOKBACK = 4;                      // groups read per look-back step
+// Words of one pass's status: tiles, then the groups' sums, then their prefixes.
+__host__ __device__ constexpr uint64_t os_groups(uint64_t tiles) { return (tiles + OS_GROUP - 1) / OS_GROUP; }
+constexpr uint64_t os_status_words(uint64_t tiles, uint64_t digits) { return (tiles + 2 * os_groups(tiles)) * digits; }
 constexpr uint32_t HIST_BLOCKS = VS_HIST_BLOCKS;
 constexpr int HIST_ITEMS = 16;       // keys per lane in flight per chunk (the kernel is latency-bound below that)
 
@@ -336,12 +401,14 @@ __device__ __forceinline__ void status_store(uint32_t* p, uint32_t v) {
 }
 
 // One pass over digits of RB bits: rank a tile, find its digits' global
-// offsets by look-back, scatter.  `status` is [nblocks][2^RB], zeroed before
-// the pass.  key_span (null: unused) is the [min, max] of values whose
+// offsets by look-back, scatter.  `status` is os_status_words(nblocks, 2^RB)
+// words ([tile or group][digit]), zeroed before the pass.  key_span (null: unused) is the [min, max] of values whose
 // differences the keys are: a pass whose digit lies above every key's
 // highest set bit is the identity, and copies its tile.
-template <typename K, int BLOCK, int ITEMS, int RB = 8>
-__global__ void __launch_bounds__(BLOCK) sort_onesweep_kernel(const K* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
+// RANGES: the last pass of a tile sort, which finds the tile ranges instead of
+// writing the keys.
+template <typename K, int BLOCK, int ITEMS, int RB, bool RANGES>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(sizeof(K) == 4 ? 4 : 3))) sort_onesweep_kernel(const K* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
                                                                    K* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
                                                                    uint32_t n_cap, const uint32_t* __restrict__ n_dev, uint32_t shift,
                                                                    const uint32_t* __restrict__ ghist, uint32_t ghist_copy_stride,
@@ -354,9 +421,8 @@ __global__ void __launch_bounds__(BLOCK) sort_onesweep_kernel(const K* __restric
     __shared__ uint32_t wave_hist[BLOCK / 64][R];
     __shared__ uint32_t digit_start[R];
     __shared__ uint32_t s_tot[BLOCK / 64];
-    __shared__ uint32_t s_gstart[R];        // where this tile's digit d starts in the output
-    __shared__ K s_keys[TILE];
-    __shared__ uint32_t s_vals[TILE];
+    __shared__ uint32_t s_off[R];           // where this tile's digit d starts in the output, less its first tile slot
+    __shared__ K s_buf[TILE];
 
     // Tile = block index.  Workgroups are dispatched in index order on each
     // XCD, so every block this one waits on (lower indices) is already
@@ -388,7 +454,8 @@ __global__ void __launch_bounds__(BLOCK) sort_onesweep_kernel(const K* __restric
 #pragma unroll
     for (uint32_t x = 0; x < HIST_COPIES; ++x) gh[x] = d < R ? ghist[(size_t)x * ghist_copy_stride + d] : 0u;
     TileRanker<K, BLOCK, ITEMS, RB> rk;
-    const uint32_t cnt = rk.count(keys_in, vals_in, base, n, shift, wave_hist);
+    rk.load(keys_in, vals_in, base, n);
+    const uint32_t cnt = rk.count(base, n, shift, wave_hist);
 
     // The tile's digit counts are published as soon as they are known, and
     // the look-back runs before the tile is reordered in LDS, so the tile's
@@ -396,20 +463,27 @@ __global__ void __launch_bounds__(BLOCK) sort_onesweep_kernel(const K* __restric
     uint32_t excl = 0;
     if (d < R) {
         uint32_t* my = status + (size_t)tile * R + d;
+        const uint32_t group = tile / OS_GROUP, ngroups = (uint32_t)os_groups(gridDim.x);
+        uint32_t* gsum = status + (size_t)gridDim.x * R + d;       // [group][R]
+        uint32_t* gpre = gsum + (size_t)ngroups * R;
         status_store(my, (tile == 0 ? OS_PREFIX : OS_AGGREGATE) | cnt);
+        __hip_atomic_fetch_add(gsum + (size_t)group * R, (1u << OS_GROUP_SHIFT) + cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (tile > 0) {
-            // Look back over predecessors LOOKBACK at a time (independent loads),
-            // newest first, summing aggregates until a prefix; a not-yet-published
-            // tile is polled again.
+            // Look back LOOKBACK predecessors at a time (independent loads),
+            // newest first, summing aggregates until a prefix or the group's
+            // first tile, then GROUP_LOOKBACK whole groups at a time; one that
+            // is not published yet is polled again.
+            const int first = (int)(group * OS_GROUP);
             int j = (int)tile - 1;
             uint32_t spins = 0;
-            while (true) {
+            bool found = false;
+            while (!found && j >= first) {
                 uint32_t st[LOOKBACK];
     #pragma unroll
                 for (int i = 0; i < LOOKBACK; ++i)
-                    st[i] = (j - i >= 0) ? status_load(status + (size_t)(j - i) * R + d) : OS_PREFIX;
+                    st[i] = (j - i >= first) ? status_load(status + (size_t)(j - i) * R + d) : OS_AGGREGATE;
                 int used = 0;
-                bool found = false, stalled = false;
+                bool stalled = false;
     #pragma unroll
                 for (int i = 0; i < LOOKBACK; ++i) {
                     if (found || stalled) continue;
@@ -419,17 +493,46 @@ __global__ void __launch_bounds__(BLOCK) sort_onesweep_kernel(const K* __restric
                     ++used;
                     found = flag == OS_PREFIX;
                 }
-                if (found) break;
                 j -= used;
-                if (stalled) {
-                    if (++spins > spin_limit) { atomicOr(err, 1u); break; }
+                if (stalled && !found) {
+                    if (++spins > spin_limit) { atomicOr(err, 1u); found = true; }
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
+            int k = (int)group - 1;
+            while (!found && k >= 0) {
+                uint32_t pre[GROUP_LOOKBACK], sum[GROUP_LOOKBACK];
+    #pragma unroll
+                for (int i = 0; i < GROUP_LOOKBACK; ++i) {
+                    pre[i] = (k - i >= 0) ? status_load(gpre + (size_t)(k - i) * R) : OS_PREFIX;
+                    sum[i] = (k - i >= 0) ? status_load(gsum + (size_t)(k - i) * R) : 0u;
+                }
+                int used = 0;
+                bool stalled = false;
+    #pragma unroll
+                for (int i = 0; i < GROUP_LOOKBACK; ++i) {
+                    if (found || stalled) continue;
+                    if (pre[i] & OS_PREFIX) {
+                        excl += pre[i] & OS_VALUE;
+                        found = true;
+                    } else if (sum[i] >> OS_GROUP_SHIFT == OS_GROUP) {
+                        excl += sum[i] & OS_GROUP_SUM;
+                        ++used;
+                    } else {
+                        stalled = true;
+                    }
+                }
+                k -= used;
+                if (stalled && !found) {
+                    if (++spins > spin_limit) { atomicOr(err, 1u); found = true; }
                     __builtin_amdgcn_s_sleep(1);
                 }
             }
             status_store(my, OS_PREFIX | (excl + cnt));
         }
+        if (tile % OS_GROUP == OS_GROUP - 1u) status_store(gpre + (size_t)group * R, OS_PREFIX | (excl + cnt));
     }
-    rk.place(wave_hist, digit_start, s_tot, s_keys, s_vals);
+    rk.starts(shift, wave_hist, digit_start, s_tot);
     // global exclusive start of digit d: sum of ghist[0..d) (block scan over R)
     {
         const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -442,35 +545,40 @@ __global__ void __launch_bounds__(BLOCK) sort_onesweep_kernel(const K* __restric
             const uint32_t t = __shfl_up(incl, o);
             if ((int)lane >= o) incl += t;
         }
-        if (lane == 63 && d < R) s_tot[wave] = incl;   // place() has finished with s_tot
+        if (lane == 63 && d < R) s_tot[wave] = incl;   // starts() has finished with s_tot
         __syncthreads();
         if (d < R) {
             uint32_t wo = 0;
             for (uint32_t w = 0; w < wave; ++w) wo += s_tot[w];
-            s_gstart[d] = excl + wo + incl - c;
+            s_off[d] = excl + wo + incl - c - digit_start[d];
         }
     }
     __syncthreads();
     const uint32_t count = min(TILE, n - base);
-    for (uint32_t i = threadIdx.x; i < count; i += BLOCK) {
-        const K k = s_keys[i];
+    const WordBuf vb = word_buf(vals_out, n);
+    const WordBuf kb = word_buf(reinterpret_cast<uint32_t*>(keys_out), sizeof(K) == 4 ? n : 0u);
+    rk.scatter(s_buf, count, [&](uint32_t i, K k) {
         const uint32_t dd = digit_rb<RB>(k, shift);
-        const uint32_t gpos = s_gstart[dd] + (i - digit_start[dd]);
-        if (gpos < n) {   // always true for consistent counts; keeps a bad count from writing out of bounds
-            if (!ranges) keys_out[gpos] = k;
-            vals_out[gpos] = s_vals[i];
-            if (ranges && (uint64_t)k < num_tiles) {
+        const uint32_t gpos = s_off[dd] + i;
+        if constexpr (sizeof(K) == 4) {
+            if (!RANGES) word_put(kb, gpos, (uint32_t)k);
+        } else {
+            if (!RANGES && gpos < n) keys_out[gpos] = k;   // always true for consistent counts; keeps a bad count from writing out of bounds
+        }
+        if constexpr (RANGES) {
+            if (gpos < n && (uint64_t)k < num_tiles) {
                 // The last pass: within a digit's run of this tile the keys are
                 // sorted (earlier passes sorted the lower bits), so a key change
                 // inside the run is a range bound; a run's first and last keys
                 // may continue in another tile's run and meet there by min / max.
                 const uint32_t t = (uint32_t)k;
                 const uint32_t run_lo = digit_start[dd], run_hi = dd < R - 1 ? digit_start[dd + 1] : count;
-                if (i == run_lo || s_keys[i - 1] != k) atomicMin(&ranges[2 * t], gpos);
-                if (i + 1 == run_hi || s_keys[i + 1] != k) atomicMax(&ranges[2 * t + 1], gpos + 1);
+                if (i == run_lo || s_buf[i - 1] != k) atomicMin(&ranges[2 * t], gpos);
+                if (i + 1 == run_hi || s_buf[i + 1] != k) atomicMax(&ranges[2 * t + 1], gpos + 1);
             }
         }
-    }
+        return gpos;
+    }, [&](uint32_t to, uint32_t v) { word_put(vb, to, v); });
 }
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -487,7 +595,7 @@ size_t sort_tmp_bytes(uint64_t n, bool key64, uint32_t radix_bits) {
     b += align_up(scan_tmp_words(nblocks * 256) * 4, 256);
     // one-sweep: histograms and per-pass tile status
     const uint64_t os_tiles = (n + OS_MIN_TILE - 1) / OS_MIN_TILE;
-    b += align_up((size_t)(HIST_COPIES * max_passes * R * 4 + 64 + max_passes * os_tiles * R * 4), 256);
+    b += align_up((size_t)(HIST_COPIES * max_passes * R * 4 + 64 + max_passes * os_status_words(os_tiles, R) * 4), 256);
     return b + 256;
 }
 
@@ -496,12 +604,19 @@ static void launch_onesweep_pass(bool small, uint32_t os_tiles, const K* src_k, 
                                  uint32_t* dv, uint32_t n, const uint32_t* n_dev, uint32_t shift, const uint32_t* gh,
                                  uint32_t gh_stride, uint32_t* status, uint32_t* err, uint32_t spin_limit,
                                  uint32_t* rng, uint32_t nt, const uint32_t* key_span, hipStream_t s) {
-    if (small)
-        sort_onesweep_kernel<K, OS_SMALL_BLOCK, OS_SMALL_ITEMS, RB><<<os_tiles, OS_SMALL_BLOCK, 0, s>>>(
-            src_k, src_v, dk, dv, n, n_dev, shift, gh, gh_stride, status, err, spin_limit, rng, nt, key_span);
-    else
-        sort_onesweep_kernel<K, OS_BLOCK, OS_ITEMS, RB><<<os_tiles, OS_BLOCK, 0, s>>>(
-            src_k, src_v, dk, dv, n, n_dev, shift, gh, gh_stride, status, err, spin_limit, rng, nt, key_span);
+    auto go = [&](auto ranges) {
+        constexpr bool R = decltype(ranges)::value;
+        if (small)
+            sort_onesweep_kernel<K, OS_SMALL_BLOCK, OS_SMALL_ITEMS, RB, R><<<os_tiles, OS_SMALL_BLOCK, 0, s>>>(
+                src_k, src_v, dk, dv, n, n_dev, shift, gh, gh_stride, status, err, spin_limit, rng, nt, key_span);
+        else
+            sort_onesweep_kernel<K, OS_BLOCK, OS_ITEMS, RB, R><<<os_tiles, OS_BLOCK, 0, s>>>(
+                src_k, src_v, dk, dv, n, n_dev, shift, gh, gh_stride, status, err, spin_limit, rng, nt, key_span);
+    };
+    if constexpr (sizeof(K) == 4) {       // 64-bit keys are never tile ids
+        if (rng) { go(std::true_type{}); return; }
+    }
+    go(std::false_type{});
 }
 
 // Digits of 8 bits, or of 7 or 9 (radix_bits, u32 keys, one-sweep schedule
@@ -534,11 +649,11 @@ static hipError_t sort_impl(const K* keys_in, const uint32_t* vals_in, K* keys_o
     const uint32_t os_tile = small ? OS_SMALL_TILE : OS_TILE;
     const uint32_t os_tiles = (n + os_tile - 1) / os_tile;
     uint32_t* ghist = reinterpret_cast<uint32_t*>(p);          // [HIST_COPIES][passes][R]
-    uint32_t* status = ghist + HIST_COPIES * passes * R + 16; // [passes][os_tiles][R]
+    uint32_t* status = ghist + HIST_COPIES * passes * R + 16; // [passes][os_status_words]
     if (onesweep) {
         hipError_t e = hipSuccess;
         if (!state_zeroed)
-            e = launch_fill_u32(ghist, 0u, (uint64_t)HIST_COPIES * passes * R + 16 + (uint64_t)passes * os_tiles * R, s);
+            e = launch_fill_u32(ghist, 0u, (uint64_t)HIST_COPIES * passes * R + 16 + passes * os_status_words(os_tiles, R), s);
         if (e != hipSuccess) return e;
         // ~4k keys per block up to HIST_BLOCKS blocks: each block ends with
         // passes x R global atomics, so a grid much wider than the data
@@ -570,7 +685,7 @@ static hipError_t sort_impl(const K* keys_in, const uint32_t* vals_in, K* keys_o
         hipError_t e;
         if (onesweep) {
             const uint32_t* gh = ghist + pass * R;
-            uint32_t* st = status + (size_t)pass * os_tiles * R;
+            uint32_t* st = status + (size_t)pass * os_status_words(os_tiles, R);
             if constexpr (sizeof(K) == 4) {
                 if (rb == 7)
                     launch_onesweep_pass<K, 7>(small, os_tiles, src_k, src_v, dk, dv, n, n_dev, shift, gh, passes * R, st,
@@ -635,7 +750,7 @@ SortZeroSpan sort_zero_span(uint32_t n, uint32_t first_bit, uint32_t end_bit, vo
     p += align_up(scan_tmp_words((uint64_t)nblocks * 256) * 4, 256);
     const uint32_t os_tile = n < OS_SMALL_N ? OS_SMALL_TILE : OS_TILE;
     const uint64_t os_tiles = (n + os_tile - 1) / os_tile;
-    return SortZeroSpan{reinterpret_cast<uint32_t*>(p), (uint64_t)HIST_COPIES * passes * R + 16 + (uint64_t)passes * os_tiles * R};
+    return SortZeroSpan{reinterpret_cast<uint32_t*>(p), (uint64_t)HIST_COPIES * passes * R + 16 + passes * os_status_words(os_tiles, R)};
 }
 
 } // namespace vs
