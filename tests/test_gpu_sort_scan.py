@@ -217,3 +217,13 @@ def test_sort_group_edges(n, span):
     ek, ev = _expected(keys, vals, 32, 0)
     np.testing.assert_array_equal(gk, ek)
     np.testing.assert_array_equal(gv, ev)
+
+
+# Prefix sums where the block size changes (2^20 elements) and at the edges of
+# 4096-element blocks, 16-byte aligned or not; wrapping mod 2^32.
+@pytest.mark.parametrize("n", [2 ** 20 - 1, 2 ** 20 + 3, 257 * 4096, 257 * 4096 + 1, 300 * 4096 - 1, 4_300_001])
+@pytest.mark.parametrize("off", [0, 1])
+def test_prefix_sum_block_edges(n, off):
+    data = np.random.default_rng(n).integers(0, 2 ** 32, n + off, dtype=np.uint64).astype(np.uint32)
+    got = va.prefix_sum(torch.from_numpy(data.view(np.int32)).cuda()[off:]).cpu().numpy().view(np.uint32)
+    np.testing.assert_array_equal(got, np.cumsum(data[off:], dtype=np.uint64).astype(np.uint32))

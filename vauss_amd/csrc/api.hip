@@ -1562,7 +1562,7 @@ extern "C" vs_status vs_prefix_sum_u32(vs_ctx* ctx, const uint32_t* in, uint32_t
     VS_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     void* tmp = nullptr;
     VS_HIP(lib_alloc(ctx, &tmp, scan_tmp_words(n) * 4, ctx->stream), "hipMallocAsync(scan tmp)");
-    hipError_t e = scan_u32(in, out, n, true, static_cast<uint32_t*>(tmp), nullptr, ctx->stream);
+    hipError_t e = scan_u32(in, out, n, true, static_cast<uint32_t*>(tmp), ctx->stream);
     lib_free(ctx, tmp);
     if (e != hipSuccess) return hip_fail(e, "prefix sum");
     return VS_OK;

@@ -1,10 +1,10 @@
 // k_scan.hip -- device-wide u32 prefix sums.
 //
 // Replaces crates/splat-train-scan (prefix_sum, lib.rs:24-83; scan_in_place,
-// lib.rs:85-96).  Reduce-then-scan over 1024-element blocks: a reduce kernel
-// writes block totals, one workgroup scans the totals, and a scan kernel
-// re-reads its block through LDS (coalesced loads, blocked per-thread
-// sequential scan, wave shuffles) and adds the block offset.
+// lib.rs:85-96).  Reduce-then-scan over blocks of 1024 or 4096 elements: a
+// reduce kernel writes block totals, one workgroup scans the totals, and a
+// scan kernel re-reads its block (four consecutive elements per thread and
+// 1024-element chunk, wave shuffles) and adds the block offset.
 #include "vs_internal.h"
 
 namespace vs {
@@ -43,11 +43,9 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t& excl, 
     return total;
 }
 
-// With a permutation `perm`, element i of the scanned sequence is in[perm[i]]
-// and its result is written to out[perm[i]] (out[i] with `in_order`, and then
-// also to out2[perm[i]] when out2 is given).  Entries at or past `perm_bound`
-// (only a corrupt permutation holds them) read as 0 and are not scattered, so
-// a bad permutation cannot index out of bounds.
+// With a permutation `perm`, element i of the scanned sequence is in[perm[i]].
+// Entries at or past `perm_bound` (only a corrupt permutation holds them) read
+// as 0, so a bad permutation cannot index out of bounds.
 __device__ __forceinline__ uint32_t scan_load(const uint32_t* __restrict__ in, const uint32_t* __restrict__ perm,
                                               uint64_t idx, uint32_t perm_bound) {
     if (!perm) return in[idx];
@@ -60,17 +58,34 @@ __device__ __forceinline__ uint64_t scan_count(uint64_t n, const uint32_t* __res
     return n_dev ? (*n_dev < n ? (uint64_t)*n_dev : n) : n;
 }
 
-__global__ void __launch_bounds__(SCAN_BLOCK) scan_reduce_kernel(const uint32_t* __restrict__ in, uint64_t n_cap,
-                                                                 uint32_t* __restrict__ sums,
-                                                                 const uint32_t* __restrict__ perm,
-                                                                 const uint32_t* __restrict__ n_dev, uint32_t perm_bound) {
-    const uint64_t n = scan_count(n_cap, n_dev);
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+// Four consecutive elements of chunk k of a block (thread t's: 4 t of the
+// chunk's 1024), as one 16-byte access where the array and the bounds allow.
+template <bool V4>
+__device__ __forceinline__ uint4 scan_load4(const uint32_t* __restrict__ in, uint64_t at, uint64_t n) {
+    if (V4 && at + 4 <= n) return *reinterpret_cast<const uint4*>(in + at);
+    uint4 q;
+    q.x = at < n ? in[at] : 0u;
+    q.y = at + 1 < n ? in[at + 1] : 0u;
+    q.z = at + 2 < n ? in[at + 2] : 0u;
+    q.w = at + 3 < n ? in[at + 3] : 0u;
+    return q;
+}
+
+// Block sums and, below, the blocks' scans, over blocks of CHUNKS x 1024
+// elements.  Bound by memory on long arrays (12 bytes an element): blocks of
+// 4096 elements with 16-byte accesses and every chunk's load in flight, from
+// SCAN_LONG elements on (30M: 48 + 28 + 53 us with 1024-element blocks and
+// dword accesses, 45 + 9 + 41 so; the middle kernel is one workgroup over the
+// block sums, a quarter as many); shorter ones keep enough blocks for the chip.
+template <int CHUNKS, bool V4>
+__global__ void __launch_bounds__(SCAN_BLOCK) scan_reduce_kernel(const uint32_t* __restrict__ in, uint64_t n,
+                                                                 uint32_t* __restrict__ sums) {
+    const uint64_t base = (uint64_t)blockIdx.x * (CHUNKS * SCAN_TILE) + threadIdx.x * 4u;
     uint32_t acc = 0;
 #pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) {
-        const uint64_t idx = base + (uint64_t)i * SCAN_BLOCK + threadIdx.x;
-        if (idx < n) acc += scan_load(in, perm, idx, perm_bound);
+    for (int k = 0; k < CHUNKS; ++k) {
+        const uint4 q = scan_load4<V4>(in, base + (uint64_t)k * SCAN_TILE, n);
+        acc += (q.x + q.y) + (q.z + q.w);
     }
     __shared__ uint32_t s_w[48];
     uint32_t excl;
@@ -78,47 +93,44 @@ __global__ void __launch_bounds__(SCAN_BLOCK) scan_reduce_kernel(const uint32_t*
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-__global__ void __launch_bounds__(SCAN_BLOCK) scan_block_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                                uint64_t n_cap, const uint32_t* __restrict__ offsets,
-                                                                int inclusive, const uint32_t* __restrict__ perm,
-                                                                const uint32_t* __restrict__ n_dev, uint32_t perm_bound,
-                                                                int in_order, uint32_t* __restrict__ out2) {
-    const uint64_t n = scan_count(n_cap, n_dev);
-    __shared__ uint32_t s_data[SCAN_TILE];
-    __shared__ uint32_t s_w[48];
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
+template <int CHUNKS, bool V4>
+__global__ void __launch_bounds__(SCAN_BLOCK) scan_block_kernel(const uint32_t* in, uint32_t* out, uint64_t n,
+                                                                const uint32_t* __restrict__ offsets, int inclusive) {
+    constexpr int WAVES = SCAN_BLOCK / 64;
+    __shared__ uint32_t s_w[CHUNKS * WAVES];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t base = (uint64_t)blockIdx.x * (CHUNKS * SCAN_TILE) + threadIdx.x * 4u;
+    uint4 q[CHUNKS];
+    uint32_t incl[CHUNKS];
 #pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) {
-        const uint32_t li = i * SCAN_BLOCK + threadIdx.x;
-        const uint64_t idx = base + li;
-        s_data[li] = (idx < n) ? scan_load(in, perm, idx, perm_bound) : 0u;
+    for (int k = 0; k < CHUNKS; ++k) q[k] = scan_load4<V4>(in, base + (uint64_t)k * SCAN_TILE, n);
+#pragma unroll
+    for (int k = 0; k < CHUNKS; ++k) {
+        incl[k] = wave_incl_scan((q[k].x + q[k].y) + (q[k].z + q[k].w), lane);
+        if (lane == 63) s_w[k * WAVES + wave] = incl[k];
     }
     __syncthreads();
-    uint32_t v[SCAN_ITEMS];
-    uint32_t acc = 0;
+    uint32_t run = offsets ? offsets[blockIdx.x] : 0u;
 #pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) { v[i] = s_data[threadIdx.x * SCAN_ITEMS + i]; acc += v[i]; }
-    uint32_t excl;
-    block_excl_scan<SCAN_BLOCK>(acc, excl, s_w);
-    uint32_t run = excl + (offsets ? offsets[blockIdx.x] : 0u);
+    for (int k = 0; k < CHUNKS; ++k) {
+        uint32_t at = run;
 #pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) {
-        const uint32_t before = run;
-        run += v[i];
-        s_data[threadIdx.x * SCAN_ITEMS + i] = inclusive ? run : before;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < SCAN_ITEMS; ++i) {
-        const uint32_t li = i * SCAN_BLOCK + threadIdx.x;
-        const uint64_t idx = base + li;
-        if (idx < n) {
-            const uint64_t j = (perm && !in_order) ? (uint64_t)perm[idx] : idx;
-            if (!perm || in_order || j < perm_bound) out[j] = s_data[li];
-            if (out2) {
-                const uint32_t k = perm[idx];
-                if (k < perm_bound) out2[k] = s_data[li];
-            }
+        for (int w = 0; w < WAVES; ++w) {
+            const uint32_t t = s_w[k * WAVES + w];
+            if (w < (int)wave) at += t;
+            run += t;
+        }
+        const uint32_t sum = (q[k].x + q[k].y) + (q[k].z + q[k].w);
+        const uint32_t e0 = at + incl[k] - sum, e1 = e0 + q[k].x, e2 = e1 + q[k].y, e3 = e2 + q[k].z;
+        const uint4 o = inclusive ? make_uint4(e1, e2, e3, e3 + q[k].w) : make_uint4(e0, e1, e2, e3);
+        const uint64_t idx = base + (uint64_t)k * SCAN_TILE;
+        if (V4 && idx + 4 <= n) {
+            *reinterpret_cast<uint4*>(out + idx) = o;
+        } else {
+            if (idx < n) out[idx] = o.x;
+            if (idx + 1 < n) out[idx + 1] = o.y;
+            if (idx + 2 < n) out[idx + 2] = o.z;
+            if (idx + 3 < n) out[idx + 3] = o.w;
         }
     }
 }
@@ -262,33 +274,26 @@ hipError_t scan_single_block(uint32_t* data, uint32_t n, bool inclusive, uint32_
     return hipGetLastError();
 }
 
-hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, bool inclusive, uint32_t* tmp,
-                    uint32_t* total_out, hipStream_t s, const uint32_t* perm, const uint32_t* n_dev,
-                    uint32_t perm_bound, bool out_in_order, uint32_t* out_scattered) {
-    const int in_order = out_in_order ? 1 : 0;
-    uint32_t* out2 = (perm && out_in_order) ? out_scattered : nullptr;
-    if (n == 0) {
-        if (total_out) return scan_single_block(tmp, 0, false, total_out, s);
-        return hipSuccess;
+constexpr uint64_t SCAN_LONG = 1u << 20;
+template <int CHUNKS, bool V4>
+static hipError_t scan_blocks_of(const uint32_t* in, uint32_t* out, uint64_t n, bool inclusive, uint32_t* tmp, hipStream_t s) {
+    const uint32_t blocks = (uint32_t)((n + CHUNKS * SCAN_TILE - 1) / (CHUNKS * SCAN_TILE));
+    if (blocks > 1) {
+        scan_reduce_kernel<CHUNKS, V4><<<blocks, SCAN_BLOCK, 0, s>>>(in, n, tmp);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        e = scan_single_block(tmp, blocks, false, nullptr, s);
+        if (e != hipSuccess) return e;
     }
-    const uint64_t blocks = (n + SCAN_TILE - 1) / SCAN_TILE;
-    if (blocks == 1) {
-        scan_block_kernel<<<1, SCAN_BLOCK, 0, s>>>(in, out, n, nullptr, inclusive ? 1 : 0, perm, n_dev, perm_bound, in_order, out2);
-        if (total_out) {
-            scan_reduce_kernel<<<1, SCAN_BLOCK, 0, s>>>(in, n, tmp, perm, n_dev, perm_bound);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-            return scan_single_block(tmp, 1, true, total_out, s);
-        }
-        return hipGetLastError();
-    }
-    scan_reduce_kernel<<<(uint32_t)blocks, SCAN_BLOCK, 0, s>>>(in, n, tmp, perm, n_dev, perm_bound);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = scan_single_block(tmp, (uint32_t)blocks, false, total_out, s);
-    if (e != hipSuccess) return e;
-    scan_block_kernel<<<(uint32_t)blocks, SCAN_BLOCK, 0, s>>>(in, out, n, tmp, inclusive ? 1 : 0, perm, n_dev, perm_bound, in_order, out2);
+    scan_block_kernel<CHUNKS, V4><<<blocks, SCAN_BLOCK, 0, s>>>(in, out, n, blocks > 1 ? tmp : nullptr, inclusive ? 1 : 0);
     return hipGetLastError();
+}
+hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, bool inclusive, uint32_t* tmp, hipStream_t s) {
+    if (n == 0) return hipSuccess;
+    const bool v4 = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0u;
+    if (n >= SCAN_LONG)
+        return v4 ? scan_blocks_of<4, true>(in, out, n, inclusive, tmp, s) : scan_blocks_of<4, false>(in, out, n, inclusive, tmp, s);
+    return v4 ? scan_blocks_of<1, true>(in, out, n, inclusive, tmp, s) : scan_blocks_of<1, false>(in, out, n, inclusive, tmp, s);
 }
 
 } // namespace vs

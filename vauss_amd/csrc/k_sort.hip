@@ -707,7 +707,7 @@ static hipError_t sort_impl(const K* keys_in, const uint32_t* vals_in, K* keys_o
             sort_upsweep_kernel<K><<<nblocks, SORT_BLOCK, 0, s>>>(src_k, n, n_dev, shift, table, nblocks);
             e = hipGetLastError();
             if (e != hipSuccess) return e;
-            e = scan_u32(table, table, (uint64_t)nblocks * 256, false, stmp, nullptr, s);
+            e = scan_u32(table, table, (uint64_t)nblocks * 256, false, stmp, s);
             if (e != hipSuccess) return e;
             sort_scatter_kernel<K><<<nblocks, SORT_BLOCK, 0, s>>>(src_k, src_v, dk, dv, n, n_dev, shift, table, nblocks);
             e = hipGetLastError();

@@ -406,24 +406,17 @@ hipError_t launch_b8_zero_rows(uint32_t* codes, uint32_t n, const uint32_t* rows
                                uint32_t row_width, hipStream_t s);
 hipError_t launch_count_mask(uint32_t w, uint32_t h, float mcx, float mcy, float mr, uint32_t* out, hipStream_t s);
 
-// Scans.  `tmp` needs scan_tmp_words(n) u32 words.  With a permutation `perm`
-// (n distinct indices below `perm_bound`, the length of `in`) the scan runs
-// along it: element i of the sequence is in[perm[i]] and its result goes to
-// out[perm[i]], or to out[i] when `out_in_order` is set, in which case
-// `out_scattered` (if given) also receives it at [perm[i]]; an index at or
-// past perm_bound reads 0 (and is not scattered).
+// Scans.  `tmp` needs scan_tmp_words(n) u32 words; `out` may be `in`.
 size_t scan_tmp_words(uint64_t n);
-// `n_dev` (device, may be null): only the first min(*n_dev, n) elements are
-// scanned, read and written.
-hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, bool inclusive, uint32_t* tmp,
-                    uint32_t* total_out, hipStream_t s, const uint32_t* perm = nullptr,
-                    const uint32_t* n_dev = nullptr, uint32_t perm_bound = 0xFFFFFFFFu, bool out_in_order = false,
-                    uint32_t* out_scattered = nullptr);
+hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, bool inclusive, uint32_t* tmp, hipStream_t s);
 hipError_t scan_single_block(uint32_t* data, uint32_t n, bool inclusive, uint32_t* total_out, hipStream_t s);
-// The same exclusive scan in one kernel by decoupled look-back, written in
-// sequence order (out[i]; with both `perm` and `out_scattered`, also
-// out_scattered[perm[i]] for the elements whose input exceeds
-// `scatter_above`).  `status` needs scan_lookback_status_words(n) words, zero
+// An exclusive scan in one kernel by decoupled look-back, written in sequence
+// order (out[i]).  With a permutation `perm` (n distinct indices below
+// `perm_bound`, the length of `in`) element i of the sequence is in[perm[i]];
+// with `out_scattered` too, out_scattered[perm[i]] also receives the results
+// of the elements whose input exceeds `scatter_above`.  An index at or past
+// perm_bound reads 0 and is not scattered.  `n_dev` (device, may be null): only
+// the first min(*n_dev, n) elements are scanned, read and written.  `status` needs scan_lookback_status_words(n) words, zero
 // on entry; a look-back that waits past `spin_limit` polls sets *err.  With
 // `write_end`, out[n] (out holds n + 1 words) receives the total.
 uint64_t scan_lookback_status_words(uint64_t n);
