@@ -97,3 +97,27 @@ def test_neural_rejections():
     with pytest.raises(ValueError):
         va.render(cam, w.img_size, t, s, o, decoder=dec, neural_degree=4)
     out.state.free()
+
+
+@pytest.mark.parametrize("n", [1, 65, 257, 530_001])
+def test_neural_backward_at_run_edges(n):
+    """Runs of 256 splats and, past 2,048 of them, of 320: a lone splat, a run's remainder, the longer runs."""
+    w = scenes.workload("c1", n)
+    sc = w.scene
+    cam = w.cameras[0].uniforms(w.img_size)
+    t, _, o = to_gpu(sc)
+    rows, W = _neural_inputs(n, 40)
+    s, dec = torch.from_numpy(rows).cuda(), torch.from_numpy(W).cuda()
+    print(f"[case] n={n}", flush=True)
+    out = va.render(cam, w.img_size, t, s, o, pass_=va.RasterPass.BACKWARD, decoder=dec, neural_degree=3)
+    ref = po.render_forward(cam, w.img_size, sc.transforms, rows, sc.raw_opacities, decoder=W, neural_degree=3)
+    v_out = l1_cotangent_np(out.out_img.cpu().numpy(), scenes.loss_target(w.img_size), None)
+    g = va.render_backward(out, t, s, o, torch.from_numpy(v_out).cuda(), decoder=dec)
+    pg = ref.project_backward(g.v_combined.cpu().numpy())
+    np.testing.assert_array_equal(g.v_coeffs.cpu().numpy().view(np.uint32), pg["v_sh"].view(np.uint32))
+    np.testing.assert_array_equal(g.v_coeffs_sq.cpu().numpy().view(np.uint32), pg["v_coeffs_sq"].view(np.uint32))
+    # sums in f32 by 64 rows, then by a run's steps (fewer than 64 of either): 128 half ulps of the absolute sum
+    bound = 128 * 2.0 ** -24 * ref.decoder_abs + 1e-12
+    err = np.abs(g.v_decoder.cpu().numpy().astype(np.float64) - pg["v_decoder"].astype(np.float64))
+    assert np.all(err <= bound), np.max(err / bound)
+    out.state.free()
