@@ -103,6 +103,23 @@ def test_sh_step_synthetic(degree, first):
     np.testing.assert_array_equal(got[0][~vis].view(np.uint16), case[0][~vis].view(np.uint16))
 
 
+@pytest.mark.parametrize("n,degree,size", [(1, 3, 1.0), (127, 2, 1.0), (128, 3, 1e-22), (129, 0, 1e-30), (300, 3, 1e22),
+                                           (300, 1, 0.0)])
+def test_sh_step_run_edges_and_division_ranges(n, degree, size):
+    """A workgroup's 128 splats and its remainder; step ratios whose terms leave (or are zeros inside) the
+    range of the reciprocal's quotient; coefficients in and below f16's normal range."""
+    print(f"[case] n={n} degree={degree} size={size}", flush=True)
+    sh, cd, rows, gsq, var, codes, scales, lr_scale = _synthetic(degree, n, 7, False)
+    rows[0], gsq[0] = 1, 1e-8
+    cd[:, :3] *= np.float32(size)
+    scales = (scales * np.float32(size)).astype(np.float32)
+    sh[::2] *= np.float16(1e-5)
+    cd[1::3, 1] = 0.0                                        # a colour channel the clamp cut off
+    case = (sh, cd, rows, gsq, var, codes, scales, lr_scale)
+    want, got = _run_both(*case, time=6)
+    _assert_same(want, got)
+
+
 @pytest.mark.parametrize("cfg,n,view", [("c2", 20_000, 0), ("c5", 20_000, 0)])
 def test_f16_render_parity(cfg, n, view):
     """Forward bit for bit, dense gradients at the contract bar, fused update
