@@ -287,3 +287,30 @@ def check_ill_conditioned_rows(got, want, vc, vc_ref, bad, sens, name, safety=10
     err = np.abs(g - w)
     assert (err <= bar).all(), (f"{name}: {int((err > bar).any(axis=1).sum())} of {int(bad.sum())} ill-conditioned "
                                 f"rows exceed their condition-scaled bar (max err / bar {float((err / bar).max()):.3g})")
+
+
+@pytest.mark.parametrize("size,n,smooth", [((16, 16), 2000, False), ((250, 241), 300, False), ((250, 241), 20_000, True),
+                                           ((500, 420), 20_000, False), ((500, 420), 3000, True),
+                                           ((600, 555), 10_000, False), ((800, 630), 10_000, False),
+                                           ((800, 630), 3000, True)],
+                         ids=lambda v: str(v).replace(" ", ""))
+def test_backward_tile_splits(size, n, smooth):
+    """One image in each range of tile counts that splits a tile's backward otherwise: a list's quarters and
+    halves (one-tile and short lists, which leave segments empty, and long ones), quadrants, quadrant pairs."""
+    sc = scenes.scene_c1(n)
+    cam = va.Camera.from_focal(float(size[0]), float(size[0]), size).uniforms(size)
+    t, s, o = to_gpu(sc)
+    pass_ = va.RasterPass.BACKWARD_SMOOTH_CUTOFF if smooth else va.RasterPass.BACKWARD
+    print(f"[case] size={size} n={n} smooth={smooth}", flush=True)
+    out = va.render(cam, size, t, s, o, pass_=pass_)
+    ref = po.render_forward(cam, size, sc.transforms, sc.sh_coeffs, sc.raw_opacities,
+                            flags=po.FLAG_BWD_INFO | (po.FLAG_SMOOTH_CUTOFF if smooth else 0))
+    img = out.out_img.cpu().numpy()
+    np.testing.assert_array_equal(img.view(np.uint32), ref.get(po.F_OUT_IMG).view(np.uint32))
+    v_out = l1_cotangent_np(img, scenes.loss_target(size))
+    g = va.render_backward(out, t, s, o, torch.from_numpy(v_out).cuda())
+    rg = ref.backward(v_out)
+    vc = g.v_combined.cpu().numpy()
+    for lo, hi, name in ((0, 2, "v_xy"), (2, 5, "v_conic"), (5, 8, "v_rgb"), (8, 9, "v_opacity"), (9, 10, "v_refine")):
+        _check_grads(vc[:, lo:hi], rg["v_combined"][:, lo:hi], name)
+    out.state.free()

@@ -24,6 +24,7 @@
 // components in registers, and the wavefront reduce-scatters them with
 // permlane swaps and DPP (no LDS traffic), so each (tile, splat) pair issues
 // one atomic instruction of at most ten lanes.
+#include <type_traits>
 #include <hip/hip_ext.h>
 #include "vs_device.h"
 #include "vs_surfel.h"
@@ -734,14 +735,21 @@ VS_DEV float reduce_scatter17(const float v[17], uint32_t lane) {
 // One 64-lane wavefront per tile; lane L owns pixel (L % 8, L / 8) of each
 // 8x8 quadrant k (k = 0..3), so the quadrant masks turn into uniform branches.
 // A lane sums its pixels' contributions in registers and the wavefront
-// reduces each splat once.  PX = 1: images of fewer than BWD_QUAD_TILES
-// tiles, which leave most SIMDs idle with one wavefront per tile, take one
-// wavefront per quadrant instead (the four of a tile on one XCD, as in the
-// forward); each reduces and adds its own sums.
-constexpr int BWD_PX = 4;
-constexpr uint32_t BWD_QUAD_TILES = 2048;
+// reduces each splat once.
+// The loop issues VALU at the chip's limit where wavefronts abound; with few
+// tiles it is one wavefront's serial walk of its list.  Smaller images spread
+// a tile over more wavefronts, at the price of a reduction each: two or one of
+// the quadrants (PX), then segments of the list (SEGS), whose wavefronts walk
+// the entries before theirs for the pixels' T and D alone, about a fifth of
+// an entry's arithmetic in the same order, so every term keeps its bits.  The lines
+// lie where the training views cross (us with PX/SEGS): 256 tiles 4/1 345,
+// 1/1 229, 1/2 209, 1/4 202; 500 tiles 1/1 298, 1/2 269, 1/4 260; 800 tiles
+// 1/1 296, 1/2 269, 1/4 284; 1024 tiles 1/1 394, 1/2 384, 1/4 411; 1200 tiles
+// 1/1 434, 2/1 502, 1/2 459; 1900 tiles 4/1 564, 2/1 451, 1/1 466; 2772 tiles
+// 4/1 296, 2/1 256, 1/1 258; 3600 tiles 4/1 624, 2/1 629.
+constexpr uint32_t BWD_SEG4_TILES = 512, BWD_SEG2_TILES = 1024, BWD_PX1_TILES = 1536, BWD_PX2_TILES = 3200;
 
-template <bool SMOOTH, int PX>
+template <bool SMOOTH, int PX, int SEGS>
 __global__ void __launch_bounds__(64) raster_bwd_kernel(RasterBwdArgs a) {
     // Per-splat values are formed once at staging, where one instruction
     // serves the 64 splats of a batch, not per (splat, wavefront) in the loop.
@@ -751,16 +759,23 @@ __global__ void __launch_bounds__(64) raster_bwd_kernel(RasterBwdArgs a) {
     __shared__ float4 s_d[BWD_BATCH];       // the conic's rows scaled to pixels: c00 W, c01 W, c01 H, c11 H
     __shared__ float s_c01[BWD_BATCH];      // c01
 
-    uint32_t slot = blockIdx.x, q0 = 0u;      // q0: the first quadrant the wavefront owns
-    if constexpr (PX == 1) {
-        const uint32_t xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
-        q0 = idx % 4;
-        slot = (idx / 4) * 8 + xcd;
-    }
+    // the parts of a tile (quadrants, then segments) on one XCD
+    constexpr uint32_t QUADS = 4 / PX, PARTS = QUADS * SEGS;
+    const uint32_t xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
+    const uint32_t q0 = idx % QUADS * PX;             // the first quadrant the wavefront owns
+    const uint32_t seg = idx / QUADS % SEGS;
+    const uint32_t slot = idx / PARTS * 8 + xcd;
     const uint32_t tile = block_tile(a.order, slot, a.num_tiles);
     if (tile >= a.num_tiles) return;   // uniform: padding blocks of the XCD mapping
-    const uint32_t lo = a.ranges[tile * 2], hi = a.ranges[tile * 2 + 1];
-    if (lo >= hi) return;   // uniform per tile
+    const uint32_t lo = a.ranges[tile * 2], end = a.ranges[tile * 2 + 1];
+    if (lo >= end) return;   // uniform per tile
+    uint32_t seg_lo = lo, hi = end;                   // the segment whose gradients the wavefront adds
+    if constexpr (SEGS > 1) {
+        const uint32_t per = ((end - lo + BWD_BATCH - 1) / BWD_BATCH + SEGS - 1) / SEGS * BWD_BATCH;
+        if (end - lo <= seg * per) return;            // uniform: fewer batches than segments
+        seg_lo = lo + seg * per;
+        hi = end - seg_lo < per ? end : seg_lo + per;
+    }
     const uint32_t tx = tile % a.tile_bw, ty = tile / a.tile_bw;
     const uint32_t lane = threadIdx.x;
     const float img_w = (float)a.img_w, img_h = (float)a.img_h;
@@ -850,6 +865,32 @@ __global__ void __launch_bounds__(64) raster_bwd_kernel(RasterBwdArgs a) {
             }
         }
         __syncthreads();
+        if constexpr (SEGS > 1) {
+            if (start < seg_lo) {                               // uniform: an earlier segment's batch, state alone
+                for (uint32_t t = 0; t < rem; ++t) {
+                    const uint32_t live = (__builtin_amdgcn_readlane(mask, t) >> q0) & alive;
+                    if (live == 0) continue;
+                    const float4 sa = s_a[t];
+                    const float4 sbv = s_b[t];
+                    const float cl_b = s_c[t].x;
+#pragma unroll
+                    for (int k = 0; k < PX; ++k) {
+                        if (!((live >> k) & 1u)) continue;      // uniform
+                        const float sigma = raster_sigma(sa.z, sa.w, sbv.x, pcx[k] - sa.x, pcy[k] - sa.y);
+                        const float alpha = __builtin_fminf(ALPHA_CAP, sbv.y * comp_exp2(-sigma));
+                        const float w_cut = SMOOTH ? cutoff_weight(alpha) : ((alpha >= ALPHA_MID) ? 1.0f : 0.0f);
+                        if (!(sigma >= 0.0f && w_cut > 0.0f)) continue;
+                        const float ae = SMOOTH ? alpha * w_cut : alpha;
+                        const float Tk = T[k], nt = Tk * (1.0f - ae);
+                        T[k] = (nt <= T_STOP) ? 0.0f : nt;
+                        if (nt <= T_STOP) continue;
+                        const float cv = __builtin_fmaf(cl_b, vb[k], __builtin_fmaf(sbv.w, vg[k], sbv.z * vr[k]));
+                        D[k] = __builtin_fmaf(-(ae * Tk), cv, D[k]);
+                    }
+                }
+                continue;
+            }
+        }
         for (uint32_t t = 0; t < rem; ++t) {
             const uint32_t live = (__builtin_amdgcn_readlane(mask, t) >> q0) & alive;
             if (live == 0) continue;                        // uniform: no quadrant reaches the cutoff
@@ -1279,11 +1320,20 @@ hipError_t launch_raster_bwd(const RasterBwdArgs& a, bool smooth, hipStream_t s,
     if (a.proj_surf) {
         k = smooth ? raster_bwd_surfel_kernel<true> : raster_bwd_surfel_kernel<false>;
         block = SURF_BWD_BLOCK;
-    } else if (a.num_tiles < BWD_QUAD_TILES) {
-        k = smooth ? raster_bwd_kernel<true, 1> : raster_bwd_kernel<false, 1>;
-        grid = dim3(4 * xcd_grid(a.num_tiles));   // four quadrant wavefronts per dispatch slot
     } else {
-        k = smooth ? raster_bwd_kernel<true, BWD_PX> : raster_bwd_kernel<false, BWD_PX>;
+        uint32_t parts = 1;
+        const auto take = [&](auto px, auto segs) {
+            k = smooth ? raster_bwd_kernel<true, px, segs> : raster_bwd_kernel<false, px, segs>;
+            parts = 4 / px * segs;
+        };
+        using std::integral_constant;
+        const integral_constant<int, 1> one; const integral_constant<int, 2> two; const integral_constant<int, 4> four;
+        if (a.num_tiles < BWD_SEG4_TILES) take(one, four);
+        else if (a.num_tiles < BWD_SEG2_TILES) take(one, two);
+        else if (a.num_tiles < BWD_PX1_TILES) take(one, one);
+        else if (a.num_tiles < BWD_PX2_TILES) take(two, one);
+        else take(four, one);
+        grid = dim3(parts * xcd_grid(a.num_tiles));
     }
     if (start) hipExtLaunchKernelGGL(k, grid, dim3(block), 0, s, start, stop, 0u, a);
     else k<<<grid, block, 0, s>>>(a);
