@@ -462,7 +462,7 @@ STAGE_OF_KERNEL = [("raster_bwd_kernel", "raster_bwd"), ("raster_fwd_kernel", "r
                    ("finalize_counts", "project"), ("compact_kernel", "emit"), ("scan_", "emit"), ("sort_", "sort"),
                    ("tile_ranges", "ranges"),
                    ("l1_cotangent", "loss"), ("loss_", "image_loss"), ("project_update", "project_update"),
-                   ("sh_step", "sh_step"), ("sh_variance", "sh_step"), ("b8_", "sh_step"),
+                   ("sh_step", "sh_step"), ("b8_", "sh_step"),
                    ("pose_", "pose_backward"), ("neural_", "neural"),
                    ("fill", "fill"), ("copyBuffer", "copy"), ("stream_", "calib"), ("elementwise", "torch")]
 
